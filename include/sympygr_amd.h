@@ -120,7 +120,9 @@ typedef struct {
                                     chunk's stencil pass overlaps the previous chunk's
                                     pointwise pass on a second stream the plan owns): plans
                                     needing more than one chunk, and plans of at least 8192
-                                    tiles without the tile queues */
+                                    tiles without the tile queues.  One-pass plans (FP64,
+                                    BSSN, standard gauge, Kreiss-Oliger) run their chunks
+                                    alternately on the two streams */
     uint32_t tile_queue;         /* 1: the stencil pass is a persistent grid fed by per-XCD
                                     tile queues (plans where at least a tenth of the tiles
                                     reach a flagged face) */
@@ -149,7 +151,9 @@ int sgr_rhs(sgr_plan *plan, double *const out[SGR_NUM_VARS], const double *const
 
 /* Same as sgr_rhs, and records events[0..1] around the stencil pass and
  * events[2..3] around the pointwise kernel on `stream` (hipEventElapsedTime
- * then gives each pass's duration).  For a plan that runs in several
+ * then gives each pass's duration).  A one-pass plan (FP64, BSSN, standard
+ * gauge, Kreiss-Oliger) has one kernel: events[0..1] bracket it, events[2..3]
+ * are recorded after it.  For a plan that runs in several
  * workspace chunks (pipelined or not), events[0..1] bracket the whole call
  * and events[2..3] are recorded at its end.  No reference counterpart: it
  * exists for measurement. */

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -100,14 +101,16 @@ int tile_shape(const sgr_block &b, int td[3])
             return fail(SGR_E_INVALID, std::string("SGR_TILE_SHAPE=") + sv +
                                            " is not a tile shape (tx,ty,tz >= 2, at most 512 points, within the "
                                            "stencil kernel's LDS arrays)");
-        return SGR_OK;
-    }
-    for (const TileShapeEntry &e : kTileTable) {
-        if (e.n[0] == b.sz[0] - 6 && e.n[1] == b.sz[1] - 6 && e.n[2] == b.sz[2] - 6) {
-            for (int k = 0; k < 3; k++) td[k] = e.t[k];
-            break;
+    } else {
+        for (const TileShapeEntry &e : kTileTable) {
+            if (e.n[0] == b.sz[0] - 6 && e.n[1] == b.sz[1] - 6 && e.n[2] == b.sz[2] - 6) {
+                for (int k = 0; k < 3; k++) td[k] = e.t[k];
+                break;
+            }
         }
     }
+    // no tile reaches beyond its block (k_rhs reads whole halo tiles)
+    for (int k = 0; k < 3; k++) td[k] = std::min(td[k], (int)b.sz[k] - 6);
     return SGR_OK;
 }
 
@@ -196,6 +199,75 @@ bool stencil_queue(uint64_t faces, uint64_t tiles)
 {
     if (const char *v = getenv("SGR_STENCIL_QUEUE")) return atoi(v) != 0;
     return tiles && faces * 10 >= tiles;
+}
+
+// Parameters whose RHS runs as the one-pass kernel k_rhs instead of the stencil
+// and pointwise passes.
+bool one_pass(const sgr_params &p)
+{
+    return p.precision == SGR_PREC_FP64 && p.formulation == SGR_FORM_BSSN && p.gauge == SGR_GAUGE_STANDARD &&
+           p.dissipation == SGR_DISS_KO;
+}
+
+// Whether one RHS call does: such parameters, and no output array shares
+// memory with an input array (k_rhs writes a point while its neighbours'
+// stencils may still read it; the two passes do not).  span: nodes of a field
+// array that the blocks reach.
+bool one_pass_call(const sgr_params &p, const FieldPtrs &in, const OutPtrs &out, const RkArgs &rk, uint64_t span)
+{
+    if (!one_pass(p)) return false;
+    auto meets = [&](const double *a, const double *b) {
+        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+        return (x < y ? y - x : x - y) < span * sizeof(double);
+    };
+    for (int f = 0; f < NF; f++)
+        for (int g = 0; g < NF; g++) {
+            if (meets(in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g])) return false;
+            if (rk.stage >= 0 && rk.stage < 3 && meets(in.p[f], rk.acc.p[g])) return false;
+        }
+    return true;
+}
+
+// Does RHS tile lt of block d come within three points of a flagged face
+// (where k_rhs takes the closure forms)?
+bool closure_tile(const BlockDesc &d, uint32_t lt)
+{
+    const int t[3] = {(int)(lt % d.ntile[0]), (int)(lt / d.ntile[0] % d.ntile[1]), (int)(lt / (d.ntile[0] * d.ntile[1]))};
+    for (int k = 0; k < 3; k++) {
+        const int o = std::min(GW + d.tdim[k] * t[k], d.n[k] - GW - d.tdim[k]);
+        if ((d.bflag >> (2 * k) & 1u && o < GW + 3) ||
+            (d.bflag >> (2 * k + 1) & 1u && o + d.tdim[k] - 1 >= d.n[k] - GW - 3))
+            return true;
+    }
+    return false;
+}
+
+// The list of one k_rhs launch over tiles t0 .. t0 + n - 1: eight consecutive
+// ranges of about equal cost (CLOSURE_COST: measured ratio of the two kinds of
+// tiles), in each the tiles without closure forms first.  Appends to `order`.
+constexpr double CLOSURE_COST = 1.4;
+TileList tile_list(const std::vector<BlockDesc> &hb, const std::vector<uint32_t> &tile_block, uint32_t t0, uint32_t n,
+                   std::vector<uint32_t> &order)
+{
+    TileList l{};
+    std::vector<bool> slow(n);
+    double total = 0.0, seen = 0.0;
+    for (uint32_t i = 0; i < n; i++) {
+        const BlockDesc &d = hb[tile_block[t0 + i]];
+        slow[i] = d.bflag && closure_tile(d, t0 + i - d.tile_base);
+        total += slow[i] ? CLOSURE_COST : 1.0;
+    }
+    uint32_t i = 0;
+    for (int x = 0; x < 8; x++) {
+        l.lo[x] = (uint32_t)order.size();
+        const uint32_t i0 = i;
+        for (; i < n && (x == 7 || seen < total * (x + 1) / 8); i++) seen += slow[i] ? CLOSURE_COST : 1.0;
+        for (int pass = 0; pass < 2; pass++)
+            for (uint32_t k = i0; k < i; k++)
+                if (slow[k] == (pass == 1)) order.push_back(t0 + k);
+    }
+    l.lo[8] = (uint32_t)order.size();
+    return l;
 }
 
 // Stencil workgroups resident at once on `device`: two per CU (LDS and
@@ -302,7 +374,7 @@ struct sgr_plan {
     sgr_params params{};
     std::vector<BlockDesc> hblocks;
     BlockDesc *d_blocks = nullptr;
-    uint32_t *d_tile_block = nullptr;   // RHS tiles: the 8^3-shaped blocks' tiles first
+    uint32_t *d_tile_block = nullptr;   // RHS tiles: the 8^3-shaped blocks' tiles first (then, one-pass plans, the lists' order)
     uint32_t *d_tile_block8 = nullptr;  // constraint-pass tiles (8^3), block order
     uint32_t ntiles = 0;
     uint32_t nfast = 0;                 // RHS tiles of 8^3-shaped blocks (tile ids 0 .. nfast-1)
@@ -331,6 +403,8 @@ struct sgr_plan {
     uint32_t cchunk_tiles = 0;   // tiles per constraint launch
     uint64_t ws_bytes = 0;
     uint64_t interior = 0;
+    std::vector<std::array<TileList, 2>> lists;  // one-pass RHS: each chunk's 8^3 tiles, and its others
+    uint64_t span = 0;           // nodes of a field array the blocks reach
     size_t wsz = sizeof(double); // bytes of one staged derivative (W)
     int nf = NF;                 // fields: NF (BSSN) or NF_CCZ4
     // ghost refresh table
@@ -424,10 +498,10 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
         }
         p->hblocks.push_back(block_desc(blocks[b], &shape[3 * b], 0, 0));
         p->interior += (uint64_t)(blocks[b].sz[0] - 6) * (blocks[b].sz[1] - 6) * (blocks[b].sz[2] - 6);
-        if (params->dissipation != SGR_DISS_KO)
-            p->lam_span = std::max<uint64_t>(p->lam_span, blocks[b].offset + (uint64_t)blocks[b].sz[0] *
-                                                                               blocks[b].sz[1] * blocks[b].sz[2]);
+        p->span = std::max<uint64_t>(p->span, blocks[b].offset + (uint64_t)blocks[b].sz[0] * blocks[b].sz[1] *
+                                                                     blocks[b].sz[2]);
     }
+    if (params->dissipation != SGR_DISS_KO) p->lam_span = p->span;
     uint64_t nt_all = 0, nt8_all = 0, faces = 0;  // RHS and constraint tiles, RHS tiles at a flagged face
     for (const BlockDesc &d : p->hblocks) {
         nt_all += (uint64_t)d.ntile[0] * d.ntile[1] * d.ntile[2];
@@ -501,6 +575,20 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
         tile_block8.insert(tile_block8.end(), nt, b);
     }
     p->ntiles = (uint32_t)tile_block.size();
+    std::vector<uint32_t> order;
+    if (one_pass(*params) && p->ntiles) {
+        const uint64_t nc = (p->ntiles + p->chunk_tiles - 1) / p->chunk_tiles;
+        for (uint64_t c = 0; c < nc; c++) {
+            std::array<TileList, 2> l{};
+            for (int k = 0; k < 2; k++) {
+                const uint64_t k0 = k ? p->nfast : 0, n = k ? p->ntiles - p->nfast : p->nfast;
+                const uint64_t a = n * c / nc, e = n * (c + 1) / nc;
+                l[k] = tile_list(p->hblocks, tile_block, (uint32_t)(k0 + a), (uint32_t)(e - a), order);
+            }
+            p->lists.push_back(l);
+        }
+        tile_block.insert(tile_block.end(), order.begin(), order.end());
+    }
     p->ntiles8 = (uint32_t)tile_block8.size();
     // optional cap on the plan's device memory (SGR_DEVICE_MEM_LIMIT_GIB):
     // a plan that would need more is refused before anything is allocated
@@ -554,6 +642,8 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
         if ((e = hipMemcpy(p->d_tile_block, tile_block.data(), tile_block.size() * sizeof(uint32_t),
                            hipMemcpyHostToDevice)) != hipSuccess)
             return bail(e, "hipMemcpy(tiles)");
+        for (auto &c : p->lists)
+            for (TileList &l : c) l.order = p->d_tile_block + p->ntiles;
         if ((e = dev_alloc((void **)&p->d_tile_block8, tile_block8.size() * sizeof(uint32_t))) != hipSuccess)
             return bail(e, "hipMalloc(constraint tiles)");
         if ((e = hipMemcpy(p->d_tile_block8, tile_block8.data(), tile_block8.size() * sizeof(uint32_t),
@@ -605,7 +695,7 @@ int sgr_plan_get_info(const sgr_plan *plan, sgr_plan_info *info)
     info->derivative_slots = rs_nslot(plan->nf) + plan->nf;
     info->chunks = plan->chunk_tiles ? (plan->ntiles + plan->chunk_tiles - 1) / plan->chunk_tiles : 0;
     info->pipelined = plan->pipe && info->chunks > 1;
-    info->tile_queue = plan->use_queue;
+    info->tile_queue = plan->use_queue && !one_pass(plan->params);
     return SGR_OK;
 }
 
@@ -647,6 +737,25 @@ static hipError_t pipelined(sgr_plan *plan, LaunchArgs a, hipStream_t stream, hi
     return e;
 }
 
+// The chunks of a one-pass plan of several: in turn on `stream`, or in a
+// pipelined plan alternately on `stream` and on plan->side.  events[0..1]
+// bracket the whole call, events[2..3] are recorded at its end.
+static hipError_t one_pass_chunks(sgr_plan *plan, LaunchArgs a, hipStream_t stream, hipEvent_t *ev)
+{
+    hipError_t e = ev ? hipEventRecord(ev[0], stream) : hipSuccess;
+    for (int q = 0; q < 4; q++) a.ev[q] = nullptr;
+    if (e == hipSuccess && plan->pipe) e = hipEventRecord(plan->pev[0], stream);
+    if (e == hipSuccess && plan->pipe) e = hipStreamWaitEvent(plan->side, plan->pev[0], 0);
+    for (size_t c = 0; e == hipSuccess && c < plan->lists.size(); c++) {
+        for (int k = 0; k < 2; k++) a.list[k] = plan->lists[c][k];
+        e = launch_rhs(a, plan->pipe && (c & 1) ? plan->side : stream);
+    }
+    if (e == hipSuccess && plan->pipe) e = hipEventRecord(plan->pev[1], plan->side);
+    if (e == hipSuccess && plan->pipe) e = hipStreamWaitEvent(stream, plan->pev[1], 0);
+    for (int q = 1; q < 4 && e == hipSuccess && ev; q++) e = hipEventRecord(ev[q], stream);
+    return e;
+}
+
 static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const double *const in[SGR_NUM_VARS],
                     hipStream_t stream, hipEvent_t *ev, const RkArgs *rk = nullptr)
 {
@@ -673,6 +782,7 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
     for (int q = 0; q < 4; q++) a.ev[q] = ev ? ev[q] : nullptr;
     a.rk.stage = -1;
     if (rk) a.rk = *rk;
+    a.fused = one_pass_call(plan->params, a.in, a.out, a.rk, plan->span);
     if (plan->params.dissipation != SGR_DISS_KO) {
         // TVB replaces the Kreiss-Oliger term: the stencil pass leaves it out
         // of the tails and k_tvb adds sigma (D_x + D_y + D_z) to them
@@ -686,7 +796,11 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
     hipGetDevice(&cur);
     if (cur != plan->device) HIP_TRY(hipSetDevice(plan->device), "hipSetDevice");
     hipError_t e = a.diss ? launch_speeds(a, stream) : hipSuccess;  // once, over every node
-    if (e == hipSuccess && plan->ntiles <= plan->chunk_tiles) {
+    if (a.fused && plan->lists.size() > 1) {
+        e = one_pass_chunks(plan, a, stream, ev);
+    } else if (e == hipSuccess && plan->ntiles <= plan->chunk_tiles) {
+        if (a.fused && plan->ntiles)
+            for (int k = 0; k < 2; k++) a.list[k] = plan->lists[0][k];
         e = launch_rhs(a, stream);
     } else if (e == hipSuccess && plan->pipe) {
         e = pipelined(plan, a, stream, ev);
@@ -1030,6 +1144,7 @@ int stage_plan(const sgr_block &b, const sgr_params *params, int device)
         d.ax[k] = axis_const(b.pmin[k], b.pmax[k], b.sz[k]);
     }
     S.plan->params = *params;
+    S.plan->span = b.offset + (uint64_t)b.sz[0] * b.sz[1] * b.sz[2];
     S.plan->use_queue = stencil_queue(face_tiles(d), S.plan->ntiles);
     *S.h_desc = d;
     HIP_TRY(hipMemcpyAsync(S.plan->d_blocks, S.h_desc, sizeof(BlockDesc), hipMemcpyHostToDevice, S.stream),
@@ -1251,6 +1366,8 @@ int sgr_rhs_block_noalloc(double *const out[SGR_NUM_VARS], const double *const i
     a.mixed = params->precision == SGR_PREC_MIXED;
     a.ccz4 = nf == NF_CCZ4;
     a.rk.stage = -1;
+    a.fused = one_pass_call(*params, a.in, a.out, a.rk, offset + (uint64_t)sz[0] * sz[1] * sz[2]);
+    for (int x = 0; x < 9; x++) a.list[is_cube8(d) ? 0 : 1].lo[x] = (uint32_t)(ntiles * x / 8);
     const hipError_t e = launch_rhs(a, stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return SGR_OK;

@@ -19,6 +19,14 @@ struct RkArgs {
     OutPtrs next;
 };
 
+// The tiles one k_rhs launch covers: entries lo[x] .. lo[x + 1] - 1 of `order`
+// (device; tile numbers relative to tile0; null: 0, 1, 2, ...) for XCD x.
+struct TileList {
+    const uint32_t *order;
+    uint32_t tile0;
+    uint32_t lo[9];
+};
+
 struct LaunchArgs {
     FieldPtrs in;
     OutPtrs out;
@@ -35,6 +43,8 @@ struct LaunchArgs {
     Params params;
     bool upwind;
     bool mixed;
+    TileList list[2];            // one-pass RHS: the launch's 8^3 tiles, and its others
+    bool fused;                  // RHS: the one-pass kernel (k_rhs, which needs no workspace), see fused_rhs
     bool ccz4;                   // the CCZ4 system (25 fields) instead of BSSN
     hipEvent_t ev[4];            // optional: start/stop of k_stencil, start/stop of k_pointwise
     RkArgs rk;                   // rk.stage < 0: plain RHS
@@ -57,7 +67,8 @@ hipError_t launch_constraints(const LaunchArgs &a, OutPtrs cout, bool psi4, hipS
 hipError_t launch_ghost_fill(OutPtrs u, int nf, const GhostPatch *patches, const GhostBox *boxes,
                              const uint32_t bstart[GHOST_CLASSES + 1], hipStream_t s);
 
-hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s);    // derivative workspace + pointwise
+// k_rhs, or k_stencil and the pointwise kernel
+hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s);
 
 // TVB dissipation: the characteristic speeds at every node (before launch_rhs)
 hipError_t launch_speeds(const LaunchArgs &a, hipStream_t s);

@@ -1,6 +1,9 @@
 // BSSN (and CCZ4) RHS kernels for gfx950 (CDNA4).
 //
-// The RHS is two passes over 8x8x8 interior tiles of every block, with a
+// The FP64 BSSN right-hand side (standard gauge, Kreiss-Oliger) is one kernel,
+// k_rhs (fused_rhs.h).  Mixed precision, CCZ4, the Rochester gauge and TVB
+// dissipation, and calls whose outputs overlap their inputs, are two passes
+// over interior tiles (8x8x8, or another shape for the block's size), with a
 // tile-major derivative workspace between them:
 //
 //   k_stencil    one 512-thread workgroup per tile.  Field by field, the 14^3
@@ -29,6 +32,8 @@
 
 #include "bssn_kernels.h"
 #include "stencils.h"
+
+#include <type_traits>
 
 #ifndef SGR_ALGEBRA_BARRIER
 #define SGR_ALGEBRA_BARRIER __builtin_amdgcn_sched_barrier(0)
@@ -801,6 +806,12 @@ __global__ __launch_bounds__(512, 4) void k_stencil(FieldPtrs in, const BlockDes
     }
 }
 
+}  // namespace sgr
+
+#include "fused_rhs.h"
+
+namespace sgr {
+
 // the BSSN system (gen/bssn_algebra_pw.inc, sympygr_amd/codegen/bssn_eqs.py)
 #define SGR_PW_NFLD NF
 #define SGR_PW_NAME k_pointwise
@@ -993,9 +1004,38 @@ static hipError_t launch_rk(const LaunchArgs &a, hipStream_t s)
     return a.rk.stage >= 0 ? launch_t<R, W, UPWIND, true>(a, s) : launch_t<R, W, UPWIND, false>(a, s);
 }
 
+// k_rhs over one list of tiles: at most one workgroup per CU, a multiple of 8
+// so that every XCD's range is served.
+template <bool UPWIND, bool GEN>
+static hipError_t launch_fused1(const LaunchArgs &a, const TileList &l, hipEvent_t e0, hipEvent_t e1, hipStream_t s)
+{
+    uint32_t most = 1;  // tiles of the longest range
+    TileRanges r;
+    for (int x = 0; x < 9; x++) r.lo[x] = l.lo[x];
+    for (int x = 0; x < 8; x++) most = r.lo[x + 1] - r.lo[x] > most ? r.lo[x + 1] - r.lo[x] : most;
+    const uint32_t cap = a.grid_cap < 16 ? 1 : a.grid_cap / 16;
+    hipExtLaunchKernelGGL((k_rhs<UPWIND, GEN>), dim3(8 * (most < cap ? most : cap)), dim3(512), 0, s, e0, e1, 0, a.in,
+                          a.out, a.blocks, a.tile_block, l.order, a.params, a.rk, l.tile0, r);
+    return hipGetLastError();
+}
+
+template <bool UPWIND>
+static hipError_t launch_fused(const LaunchArgs &a, hipStream_t s)
+{
+    const bool fast = a.list[0].lo[8] > a.list[0].lo[0], gen = a.list[1].lo[8] > a.list[1].lo[0];
+    hipError_t e = hipSuccess;
+    if (fast) e = launch_fused1<UPWIND, false>(a, a.list[0], a.ev[0], gen ? nullptr : a.ev[1], s);
+    if (e == hipSuccess && gen) e = launch_fused1<UPWIND, true>(a, a.list[1], fast ? nullptr : a.ev[0], a.ev[1], s);
+    for (int q = 2; q < 4; q++)
+        if (e == hipSuccess && a.ev[q]) e = hipEventRecord(a.ev[q], s);
+    return e;
+}
+
 hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s)
 {
     if (a.ntiles == 0) return hipSuccess;
+    if (a.fused)
+        return a.only == 2 ? hipSuccess : a.upwind ? launch_fused<true>(a, s) : launch_fused<false>(a, s);
     if (a.mixed) return a.upwind ? launch_rk<float, float, true>(a, s) : launch_rk<float, float, false>(a, s);
     return a.upwind ? launch_rk<double, double, true>(a, s) : launch_rk<double, double, false>(a, s);
 }

@@ -1,0 +1,95 @@
+"""The one-pass right-hand side (FP64, BSSN, standard gauge, Kreiss-Oliger) at
+the sizes where its tiling can go wrong: blocks smaller than a tile, one tile,
+one point more or less, axes of different sizes, flagged faces whose closures
+reach into one or two tiles, and more tiles than workgroups; and calls whose
+outputs share memory with the inputs, which take the two passes.  Against the
+CPU oracle at the FP64 bar, 1e-12 normwise per field (both evaluate the same
+stencils bit for bit; the algebra differs in rounding only)."""
+import numpy as np
+import pytest
+
+from helpers import interior, normwise
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(7, 7, 7), (7, 9, 16), (8, 8, 8), (9, 8, 7), (15, 16, 17), (13, 33, 8), (10, 11, 12)]
+
+
+def _block(n, bflag, seed):
+    from sympygr_amd import data
+    bl = data.BlockList()
+    sz = tuple(k + 6 for k in n)
+    pmin = (-0.6, -0.5, -0.7)
+    bl.add(sz, pmin, tuple(p + 0.05 * (s - 1) for p, s in zip(pmin, sz)), bflag)
+    m = max(sz)
+    u = data.perturbed_flat_block(seed=seed, n=m, amp=1e-2, pmin=pmin, pmax=tuple(p + 0.05 * (m - 1) for p in pmin))
+    u = u.reshape(24, m, m, m)[:, :sz[2], :sz[1], :sz[0]].reshape(24, -1)
+    return bl, np.ascontiguousarray(u)
+
+
+def _oracle(bl, u, adv):
+    import pyoracle as po
+    return po.rhs_block(u, bl.sz[0], bl.pmin[0], bl.pmax[0], bl.bflag[0],
+                        po.make_params(upwind=adv == "upwind", ko_sigma=0.1))
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("bflag,adv", [(0, "upwind"), (63, "upwind"), (38, "centred")])
+def test_edge_sizes_against_oracle(n, bflag, adv):
+    import torch
+    import sympygr_amd as sgr
+    bl, u = _block(n, bflag, 3 + n[0])
+    prm = sgr.params(adv=adv, ko_sigma=0.1)
+    du = torch.from_numpy(u).cuda()
+    ref = interior(_oracle(bl, u, adv), bl.sz[0])
+    out = torch.full_like(du, 5.0)
+    sgr.Plan(bl, prm).rhs(out, du)
+    one = torch.full_like(du, 5.0)
+    sgr.rhs_block_noalloc(one, du, 0, bl.pmin[0], bl.pmax[0], bl.sz[0], bflag, prm)
+    torch.cuda.synchronize()
+    assert torch.equal(one, out)
+    got = out.cpu().numpy()
+    assert normwise(interior(got, bl.sz[0]), ref).max() <= 1e-12
+    ghosts = np.ones(got[0].size, dtype=bool).reshape(bl.sz[0][::-1])
+    ghosts[3:-3, 3:-3, 3:-3] = False
+    assert (got[:, ghosts.reshape(-1)] == 5.0).all()
+
+
+def test_outputs_over_inputs():
+    """In place: the two-pass kernels, same result to rounding."""
+    import torch
+    import sympygr_amd as sgr
+    bl, u = _block((13, 16, 9), 21, 8)
+    plan = sgr.Plan(bl, sgr.params(adv="upwind", ko_sigma=0.1))
+    du = torch.from_numpy(u).cuda()
+    plan.rhs(du, du)
+    torch.cuda.synchronize()
+    ref = interior(_oracle(bl, u, "upwind"), bl.sz[0])
+    assert normwise(interior(du.cpu().numpy(), bl.sz[0]), ref).max() <= 1e-12
+
+
+@pytest.mark.parametrize("faces", [False, True])
+def test_many_tiles_equal_single_blocks(faces):
+    """More tiles than workgroups (several tiles each, fetched ahead across
+    tile boundaries, both kinds of tiles in one list, 8^3 and general shapes):
+    every block equals the same block evaluated by itself, bit for bit."""
+    import torch
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    bl = data.BlockList()
+    for b in range(80):
+        n = (16, 17, 24, 13)[b % 4] + 6
+        lo = -1.0 + 0.02 * b
+        bl.add((n, n, n), (lo, -0.5, -0.7), (lo + 0.04 * (n - 1), -0.5 + 0.04 * (n - 1), -0.7 + 0.04 * (n - 1)),
+               (b * 7) & 63 if faces else 0)
+    u = data.fill_blocks(bl, backend="torch", device="cuda", kind="perturbed", seed=5, amp=1e-2, lo=-1.0, L=2.0)
+    prm = sgr.params(adv="upwind", ko_sigma=0.1)
+    out = torch.full_like(u, 5.0)
+    plan = sgr.Plan(bl, prm)
+    assert plan.info().tiles > 512
+    plan.rhs(out, u)
+    ref = torch.full_like(u, 5.0)
+    for b in range(len(bl)):
+        sgr.rhs_block(ref, u, bl.offsets[b], bl.pmin[b], bl.pmax[b], bl.sz[b], bl.bflag[b], prm)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
