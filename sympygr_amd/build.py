@@ -12,6 +12,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -19,10 +21,10 @@ CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libsympygr_amd.so")
 ARCH = os.environ.get("SGR_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["bssn_kernels.hip", "bssn_capi.hip", "ghost_table.cpp", "bssnrhs_dropin.cpp"]
+SOURCES = ["bssn_kernels.hip", "one_pass.hip", "bssn_capi.hip", "ghost_table.cpp", "bssnrhs_dropin.cpp"]
 
 HIPCC_FLAGS = [
-    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
+    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     # packed FP32 (v_pk_*_f32) is kept off for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
@@ -38,19 +40,27 @@ def hipcc():
 
 
 def build(resource_usage=False, verbose=False):
+    """Compile every source (side by side) and link the library."""
     srcs = [os.path.join(CSRC, s) for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
-    tmp = LIB + ".tmp"
-    cmd = [hipcc()] + HIPCC_FLAGS + ["-o", tmp] + srcs
-    if resource_usage:
-        cmd.insert(1, "-Rpass-analysis=kernel-resource-usage")
-    if verbose:
-        print(" ".join(cmd))
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("hipcc failed")
+    extra = ["-Rpass-analysis=kernel-resource-usage"] if resource_usage else []
+
+    def run(cmd):
+        if verbose:
+            print(" ".join(cmd))
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            sys.stderr.write(r.stdout + r.stderr)
+            raise RuntimeError("hipcc failed")
+        return r.stderr if resource_usage else ""
+
+    with tempfile.TemporaryDirectory() as d:
+        objs = [os.path.join(d, os.path.basename(s) + ".o") for s in srcs]
+        with ThreadPoolExecutor(len(srcs)) as ex:
+            out = list(ex.map(lambda so: run([hipcc()] + extra + HIPCC_FLAGS + ["-c", so[0], "-o", so[1]]), zip(srcs, objs)))
+        tmp = LIB + ".tmp"
+        run([hipcc()] + HIPCC_FLAGS + ["-shared", "-o", tmp] + objs)
     os.replace(tmp, LIB)
-    return r.stderr if resource_usage else ""
+    return "".join(out)
 
 
 if __name__ == "__main__":

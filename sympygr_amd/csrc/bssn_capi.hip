@@ -245,7 +245,7 @@ bool closure_tile(const BlockDesc &d, uint32_t lt)
 // The list of one k_rhs launch over tiles t0 .. t0 + n - 1: eight consecutive
 // ranges of about equal cost (CLOSURE_COST: measured ratio of the two kinds of
 // tiles), in each the tiles without closure forms first.  Appends to `order`.
-constexpr double CLOSURE_COST = 1.4;
+constexpr double CLOSURE_COST = 1.9;
 TileList tile_list(const std::vector<BlockDesc> &hb, const std::vector<uint32_t> &tile_block, uint32_t t0, uint32_t n,
                    std::vector<uint32_t> &order)
 {

@@ -67,6 +67,9 @@ hipError_t launch_constraints(const LaunchArgs &a, OutPtrs cout, bool psi4, hipS
 hipError_t launch_ghost_fill(OutPtrs u, int nf, const GhostPatch *patches, const GhostBox *boxes,
                              const uint32_t bstart[GHOST_CLASSES + 1], hipStream_t s);
 
+// the RHS as one kernel (k_rhs, one_pass.hip)
+hipError_t launch_one_pass(const LaunchArgs &a, hipStream_t s);
+
 // k_rhs, or k_stencil and the pointwise kernel
 hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s);
 
