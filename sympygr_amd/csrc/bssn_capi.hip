@@ -209,6 +209,13 @@ bool one_pass(const sgr_params &p)
            p.dissipation == SGR_DISS_KO;
 }
 
+// Do two arrays of `span` values share memory?
+bool arrays_meet(const double *a, const double *b, uint64_t span)
+{
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return (x < y ? y - x : x - y) < span * sizeof(double);
+}
+
 // Whether one RHS call does: such parameters, and no output array shares
 // memory with an input array (k_rhs writes a point while its neighbours'
 // stencils may still read it; the two passes do not).  span: nodes of a field
@@ -216,10 +223,7 @@ bool one_pass(const sgr_params &p)
 bool one_pass_call(const sgr_params &p, const FieldPtrs &in, const OutPtrs &out, const RkArgs &rk, uint64_t span)
 {
     if (!one_pass(p)) return false;
-    auto meets = [&](const double *a, const double *b) {
-        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-        return (x < y ? y - x : x - y) < span * sizeof(double);
-    };
+    auto meets = [&](const double *a, const double *b) { return arrays_meet(a, b, span); };
     for (int f = 0; f < NF; f++)
         for (int g = 0; g < NF; g++) {
             if (meets(in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g])) return false;
@@ -403,6 +407,7 @@ struct sgr_plan {
     uint32_t cchunk_tiles = 0;   // tiles per constraint launch
     uint64_t ws_bytes = 0;
     uint64_t interior = 0;
+    std::array<TileList, 2> all{};  // one-pass constraints: the plan's 8^3 tiles, and its others
     std::vector<std::array<TileList, 2>> lists;  // one-pass RHS: each chunk's 8^3 tiles, and its others
     uint64_t span = 0;           // nodes of a field array the blocks reach
     size_t wsz = sizeof(double); // bytes of one staged derivative (W)
@@ -576,9 +581,14 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
     }
     p->ntiles = (uint32_t)tile_block.size();
     std::vector<uint32_t> order;
+    if (p->ntiles) {
+        p->all[0] = tile_list(p->hblocks, tile_block, 0, p->nfast, order);
+        p->all[1] = tile_list(p->hblocks, tile_block, p->nfast, p->ntiles - p->nfast, order);
+    }
     if (one_pass(*params) && p->ntiles) {
         const uint64_t nc = (p->ntiles + p->chunk_tiles - 1) / p->chunk_tiles;
-        for (uint64_t c = 0; c < nc; c++) {
+        if (nc == 1) p->lists.push_back(p->all);
+        for (uint64_t c = 0; nc > 1 && c < nc; c++) {
             std::array<TileList, 2> l{};
             for (int k = 0; k < 2; k++) {
                 const uint64_t k0 = k ? p->nfast : 0, n = k ? p->ntiles - p->nfast : p->nfast;
@@ -587,8 +597,8 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
             }
             p->lists.push_back(l);
         }
-        tile_block.insert(tile_block.end(), order.begin(), order.end());
     }
+    tile_block.insert(tile_block.end(), order.begin(), order.end());
     p->ntiles8 = (uint32_t)tile_block8.size();
     // optional cap on the plan's device memory (SGR_DEVICE_MEM_LIMIT_GIB):
     // a plan that would need more is refused before anything is allocated
@@ -642,6 +652,7 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
         if ((e = hipMemcpy(p->d_tile_block, tile_block.data(), tile_block.size() * sizeof(uint32_t),
                            hipMemcpyHostToDevice)) != hipSuccess)
             return bail(e, "hipMemcpy(tiles)");
+        for (TileList &l : p->all) l.order = p->d_tile_block + p->ntiles;
         for (auto &c : p->lists)
             for (TileList &l : c) l.order = p->d_tile_block + p->ntiles;
         if ((e = dev_alloc((void **)&p->d_tile_block8, tile_block8.size() * sizeof(uint32_t))) != hipSuccess)
@@ -850,8 +861,15 @@ static int constraints_impl(sgr_plan *plan, const double *const in[SGR_NUM_VARS]
         if (!out[c]) return fail(SGR_E_INVALID, "null constraint pointer");
         co.p[c] = out[c];
     }
+    // one kernel, unless an output shares memory with an input: its points are
+    // written while their neighbours' stencils may still read them
+    bool fused = true;
+    for (int f = 0; f < NF; f++)
+        for (int c = 0; c < (psi4 ? 6 : 4); c++) fused = fused && !arrays_meet(in[f], out[c], plan->span);
     a.blocks = plan->d_blocks;
-    a.tile_block = plan->d_tile_block8;
+    a.tile_block = fused ? plan->d_tile_block : plan->d_tile_block8;
+    a.grid_cap = plan->grid_cap;
+    for (int k = 0; k < 2; k++) a.list[k] = plan->all[k];
     a.ntiles = plan->ntiles8;
     a.ws = plan->d_ws;
     a.wsK = (double *)((char *)plan->d_ws + (uint64_t)plan->cchunk_tiles * TILE_PTS * NSLOT * plan->wsz);
@@ -862,7 +880,8 @@ static int constraints_impl(sgr_plan *plan, const double *const in[SGR_NUM_VARS]
     hipGetDevice(&cur);
     if (cur != plan->device) HIP_TRY(hipSetDevice(plan->device), "hipSetDevice");
     hipError_t e = hipSuccess;
-    for (uint32_t t0 = 0; e == hipSuccess && t0 < plan->ntiles8; t0 += plan->cchunk_tiles) {
+    if (fused) e = launch_monitor(a, co, psi4, stream);
+    for (uint32_t t0 = 0; !fused && e == hipSuccess && t0 < plan->ntiles8; t0 += plan->cchunk_tiles) {
         a.tile0 = t0;
         a.ntiles = plan->ntiles8 - t0 < plan->cchunk_tiles ? plan->ntiles8 - t0 : plan->cchunk_tiles;
         e = launch_constraints(a, co, psi4, stream);

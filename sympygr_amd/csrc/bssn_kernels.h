@@ -63,6 +63,9 @@ struct LaunchArgs {
 // Re/Im Psi4 (cout[4], cout[5]); uses the workspace.
 hipError_t launch_constraints(const LaunchArgs &a, OutPtrs cout, bool psi4, hipStream_t s);
 
+// the same as one kernel (k_monitor) over a.list, without the workspace
+hipError_t launch_monitor(const LaunchArgs &a, const OutPtrs &cout, bool psi4, hipStream_t s);
+
 // boxes sorted by class: class c occupies [bstart[c], bstart[c+1])
 hipError_t launch_ghost_fill(OutPtrs u, int nf, const GhostPatch *patches, const GhostBox *boxes,
                              const uint32_t bstart[GHOST_CLASSES + 1], hipStream_t s);

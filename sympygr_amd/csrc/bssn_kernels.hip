@@ -25,8 +25,9 @@
 //                writes the RHS or the fused RK4 stage update.
 //
 // Both read the block table and a tile->block map, so one launch covers any
-// mix of block sizes.  k_derivs + k_constraints are the constraint pass (the
-// stencil kernel of the earlier layout, which stages every first derivative);
+// mix of block sizes.  k_derivs + k_constraints are the constraint pass of
+// calls whose outputs share memory with the inputs (the stencil kernel of the
+// earlier layout, which stages every first derivative; monitor.hip otherwise);
 // k_ghost_sep / k_ghost_copy refresh ghost nodes from the owning blocks.
 #include <hip/hip_ext.h>
 
