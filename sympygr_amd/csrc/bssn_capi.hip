@@ -205,8 +205,7 @@ bool stencil_queue(uint64_t faces, uint64_t tiles)
 // and pointwise passes.
 bool one_pass(const sgr_params &p)
 {
-    return p.precision == SGR_PREC_FP64 && p.formulation == SGR_FORM_BSSN && p.gauge == SGR_GAUGE_STANDARD &&
-           p.dissipation == SGR_DISS_KO;
+    return p.precision == SGR_PREC_FP64 && p.gauge == SGR_GAUGE_STANDARD && p.dissipation == SGR_DISS_KO;
 }
 
 // Do two arrays of `span` values share memory?
@@ -224,8 +223,9 @@ bool one_pass_call(const sgr_params &p, const FieldPtrs &in, const OutPtrs &out,
 {
     if (!one_pass(p)) return false;
     auto meets = [&](const double *a, const double *b) { return arrays_meet(a, b, span); };
-    for (int f = 0; f < NF; f++)
-        for (int g = 0; g < NF; g++) {
+    const int nf = p.formulation == SGR_FORM_CCZ4 ? NF_CCZ4 : NF;
+    for (int f = 0; f < nf; f++)
+        for (int g = 0; g < nf; g++) {
             if (meets(in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g])) return false;
             if (rk.stage >= 0 && rk.stage < 3 && meets(in.p[f], rk.acc.p[g])) return false;
         }

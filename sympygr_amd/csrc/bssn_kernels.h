@@ -20,10 +20,9 @@ struct RkArgs {
 };
 
 // The tiles one k_rhs launch covers: entries lo[x] .. lo[x + 1] - 1 of `order`
-// (device; tile numbers relative to tile0; null: 0, 1, 2, ...) for XCD x.
+// (device; null: 0, 1, 2, ...) for XCD x.
 struct TileList {
     const uint32_t *order;
-    uint32_t tile0;
     uint32_t lo[9];
 };
 
@@ -72,6 +71,9 @@ hipError_t launch_ghost_fill(OutPtrs u, int nf, const GhostPatch *patches, const
 
 // the RHS as one kernel (k_rhs, one_pass.hip)
 hipError_t launch_one_pass(const LaunchArgs &a, hipStream_t s);
+
+// the CCZ4 RHS as one kernel (k_ccz4_rhs, one_pass_ccz4.hip)
+hipError_t launch_one_pass_ccz4(const LaunchArgs &a, hipStream_t s);
 
 // k_rhs, or k_stencil and the pointwise kernel
 hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s);

@@ -849,8 +849,7 @@ static hipError_t launch_rk(const LaunchArgs &a, hipStream_t s)
 hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s)
 {
     if (a.ntiles == 0) return hipSuccess;
-    if (a.fused)
-        return launch_one_pass(a, s);
+    if (a.fused) return a.ccz4 ? launch_one_pass_ccz4(a, s) : launch_one_pass(a, s);
     if (a.mixed) return a.upwind ? launch_rk<float, float, true>(a, s) : launch_rk<float, float, false>(a, s);
     return a.upwind ? launch_rk<double, double, true>(a, s) : launch_rk<double, double, false>(a, s);
 }

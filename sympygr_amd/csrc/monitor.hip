@@ -11,22 +11,19 @@ namespace sgr {
 template <bool PSI4, bool GEN, bool ROUND>
 __global__ __launch_bounds__(512, 2) void k_monitor(FieldPtrs in, OutPtrs out, const BlockDesc *__restrict__ blocks,
                                                     const uint32_t *__restrict__ tile_block,
-                                                    const uint32_t *__restrict__ order, uint32_t tile0, TileRanges ranges)
+                                                    const uint32_t *__restrict__ order, TileRanges ranges)
 {
     one_pass<PSI4 ? Pass::PSI4 : Pass::CONSTRAINTS, false, GEN, false, ROUND>(in, out, blocks, tile_block, order, Params{},
-                                                                              RkArgs{}, tile0, ranges);
+                                                                              RkArgs{}, ranges);
 }
 
 template <bool PSI4, bool GEN, bool ROUND>
 static hipError_t launch_list(const LaunchArgs &a, const OutPtrs &out, const TileList &l, hipStream_t s)
 {
-    uint32_t most = 1;  // tiles of the longest range
     TileRanges r;
-    for (int x = 0; x < 9; x++) r.lo[x] = l.lo[x];
-    for (int x = 0; x < 8; x++) most = r.lo[x + 1] - r.lo[x] > most ? r.lo[x + 1] - r.lo[x] : most;
-    const uint32_t cap = a.grid_cap < 16 ? 1 : a.grid_cap / 16;
-    hipLaunchKernelGGL((k_monitor<PSI4, GEN, ROUND>), dim3(8 * (most < cap ? most : cap)), dim3(512), 0, s, a.in, out,
-                       a.blocks, a.tile_block, l.order, l.tile0, r);
+    const uint32_t grid = list_grid(l, a.grid_cap, r);
+    hipLaunchKernelGGL((k_monitor<PSI4, GEN, ROUND>), dim3(grid), dim3(512), 0, s, a.in, out,
+                       a.blocks, a.tile_block, l.order, r);
     return hipGetLastError();
 }
 

@@ -29,6 +29,11 @@
 
 namespace sgr {
 
+// Products fused into sums where the source says so, statement by statement (the
+// compiler's own choice differs between the kernels of the two tile shapes, whose
+// results have to be the same bits).
+#pragma clang fp contract(on)
+
 // Keeps the scheduler from mixing the steps of a fold: their intermediate
 // values then die before the next step's are formed.
 #define SGR_STEP __builtin_amdgcn_sched_barrier(0)
@@ -475,7 +480,7 @@ struct TileRanges {
 // flagged face run their own copy of the code, the only one with the closure
 // forms; `order` lists each range's other tiles first, so that a CU works in
 // one copy at a time (both do not fit its instruction cache).
-// order: tile numbers relative to tile0, or null for 0, 1, 2, ...
+// order: the list's tile numbers, or null for 0, 1, 2, ...
 // RK: an RK stage's update instead of the plain RHS (rk.stage >= 0).  ROUND
 // (constraints): derivatives rounded to float where the two passes stage them.
 // The kernels (k_rhs, ...) are this function; out holds the equations or the
@@ -483,7 +488,7 @@ struct TileRanges {
 template <Pass PASS, bool UPWIND, bool GEN, bool RK, bool ROUND>
 __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out, const BlockDesc *__restrict__ blocks,
                                          const uint32_t *__restrict__ tile_block, const uint32_t *__restrict__ order,
-                                         const Params &P, const RkArgs &rk, uint32_t tile0, const TileRanges &ranges)
+                                         const Params &P, const RkArgs &rk, const TileRanges &ranges)
 {
     typedef Fields<PASS> F;
     constexpr bool MONITOR = F::MONITOR, CCZ4 = F::CCZ4;
@@ -1193,6 +1198,55 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
         if (m >= end) break;
         tile = next, nb = nnext, D = Dnext, tc = tnc;
     }
+}
+
+template <Pass PASS, bool UPWIND, bool GEN, bool RK>
+__global__ __launch_bounds__(512, 2) void k_rhs(FieldPtrs in, OutPtrs out, const BlockDesc *__restrict__ blocks,
+                                                const uint32_t *__restrict__ tile_block,
+                                                const uint32_t *__restrict__ order, Params P, RkArgs rk,
+                                                TileRanges ranges)
+{
+    one_pass<PASS, UPWIND, GEN, RK, false>(in, out, blocks, tile_block, order, P, rk, ranges);
+}
+
+// A launch over one list of tiles: its ranges, and at most one workgroup per
+// CU, a multiple of 8 so that every XCD's range is served.
+inline uint32_t list_grid(const TileList &l, uint32_t grid_cap, TileRanges &r)
+{
+    uint32_t most = 1;  // tiles of the longest range
+    for (int x = 0; x < 9; x++) r.lo[x] = l.lo[x];
+    for (int x = 0; x < 8; x++) most = r.lo[x + 1] - r.lo[x] > most ? r.lo[x + 1] - r.lo[x] : most;
+    const uint32_t cap = grid_cap < 16 ? 1 : grid_cap / 16;
+    return 8 * (most < cap ? most : cap);
+}
+
+template <Pass PASS, bool UPWIND, bool GEN, bool RK>
+static hipError_t launch_list(const LaunchArgs &a, const TileList &l, hipEvent_t e0, hipEvent_t e1, hipStream_t s)
+{
+    TileRanges r;
+    const uint32_t grid = list_grid(l, a.grid_cap, r);
+    hipExtLaunchKernelGGL((k_rhs<PASS, UPWIND, GEN, RK>), dim3(grid), dim3(512), 0, s, e0, e1, 0, a.in, a.out, a.blocks,
+                          a.tile_block, l.order, a.params, a.rk, r);
+    return hipGetLastError();
+}
+
+template <Pass PASS, bool UPWIND, bool RK>
+static hipError_t launch_lists(const LaunchArgs &a, hipStream_t s)
+{
+    const bool fast = a.list[0].lo[8] > a.list[0].lo[0], gen = a.list[1].lo[8] > a.list[1].lo[0];
+    hipError_t e = hipSuccess;
+    if (fast) e = launch_list<PASS, UPWIND, false, RK>(a, a.list[0], a.ev[0], gen ? nullptr : a.ev[1], s);
+    if (e == hipSuccess && gen) e = launch_list<PASS, UPWIND, true, RK>(a, a.list[1], fast ? nullptr : a.ev[0], a.ev[1], s);
+    for (int q = 2; q < 4; q++)
+        if (e == hipSuccess && a.ev[q]) e = hipEventRecord(a.ev[q], s);
+    return e;
+}
+
+template <Pass PASS>
+static hipError_t launch_pass(const LaunchArgs &a, hipStream_t s)
+{
+    if (a.rk.stage >= 0) return a.upwind ? launch_lists<PASS, true, true>(a, s) : launch_lists<PASS, false, true>(a, s);
+    return a.upwind ? launch_lists<PASS, true, false>(a, s) : launch_lists<PASS, false, false>(a, s);
 }
 
 }  // namespace sgr

@@ -93,3 +93,49 @@ def test_many_tiles_equal_single_blocks(faces):
         sgr.rhs_block(ref, u, bl.offsets[b], bl.pmin[b], bl.pmax[b], bl.sz[b], bl.bflag[b], prm)
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("bflag,adv", [(0, "upwind"), (63, "upwind"), (38, "centred")])
+def test_ccz4_edge_sizes_against_oracle(n, bflag, adv):
+    """The CCZ4 form of the kernel (25 fields, the divergence of Gamma-hat added
+    to the K and Theta equations after their own fields) at the same sizes and
+    bar, and a first RK stage from it: u + dt/2 rhs and rhs dt/6 + u."""
+    import pyoracle as po
+    import torch
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    kappa = (0.02, 0.1, 0.5)
+    bl, _ = _block(n, bflag, 0)
+    m = max(bl.sz[0])
+    cube = data.BlockList()
+    cube.add((m,) * 3, bl.pmin[0], tuple(p + 0.05 * (m - 1) for p in bl.pmin[0]), 0)
+    u = data.fill_blocks(cube, kind="ccz4", seed=4, amp=1e-2, lo=-1.05, L=2.1)
+    s = bl.sz[0]
+    u = np.ascontiguousarray(u.reshape(25, m, m, m)[:, :s[2], :s[1], :s[0]].reshape(25, -1))
+    prm = sgr.params(adv=adv, ko_sigma=0.1, formulation="ccz4", kappa=kappa)
+    ref = po.rhs_block(u, s, bl.pmin[0], bl.pmax[0], bflag,
+                       po.make_params(upwind=adv == "upwind", ko_sigma=0.1, ccz4=True, kappa=kappa))
+    du = torch.from_numpy(u).cuda()
+    out = torch.full_like(du, 5.0)
+    plan = sgr.Plan(bl, prm)
+    plan.rhs(out, du)
+    one = torch.full_like(du, 5.0)
+    sgr.rhs_block_noalloc(one, du, 0, bl.pmin[0], bl.pmax[0], s, bflag, prm)
+    acc, nxt = torch.zeros_like(du), torch.zeros_like(du)
+    dt = 0.0625
+    plan.rk4_stage(0, dt, du, du, acc, nxt)
+    torch.cuda.synchronize()
+    assert torch.equal(one, out)
+    inner = (slice(None), slice(3, -3), slice(3, -3), slice(3, -3))
+
+    def of(a):
+        return np.asarray(a).reshape(25, s[2], s[1], s[0])[inner].reshape(25, -1)
+    got, r, u0 = of(out.cpu()), of(ref), of(u)
+    scale = np.abs(r).max(axis=1) + 1e-300
+    assert (np.abs(got - r).max(axis=1) / scale).max() <= 1e-12
+    # one rounding of the product, one of the sum
+    eps = 2.0 ** -52
+    for a, w in ((nxt, 0.5 * dt), (acc, dt / 6.0)):
+        assert (np.abs(of(a.cpu()) - (u0 + w * got)) <= 2 * eps * (np.abs(u0) + np.abs(w * got))).all()
+    assert (out.cpu().reshape(25, s[2], s[1], s[0])[:, :3] == 5.0).all()
