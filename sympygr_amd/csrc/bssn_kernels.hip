@@ -1006,7 +1006,7 @@ __global__ __launch_bounds__(256) void k_ghost_sep(OutPtrs u, int nf, const Ghos
     __shared__ double wxs[GHOST_BOX_MAX * NX], wys[GHOST_BOX_MAX * NY], wzs[GHOST_BOX_MAX * NZ];
     __shared__ int px[GHOST_BOX_MAX], ry0[GHOST_BOX_MAX], rz0[GHOST_BOX_MAX];
     __shared__ int rowy[GHOST_ROWS_MAX], rowz[GHOST_ROWS_MAX];  // source y (z) node of each row
-    const GhostBox bx = boxes[blockIdx.x];
+    const GhostBox bx = boxes[xcd_remap(blockIdx.x, gridDim.x)];
     const GhostPatch g = patches[bx.patch];
     const int ex = bx.e[0], ey = bx.e[1], ez = bx.e[2];
     const int Ry = ghost_rows(bx.lo[1], ey, g.rel[1], g.ht[1], g.hs[1], g.sm[1], NY);
@@ -1095,7 +1095,7 @@ __global__ __launch_bounds__(256) void k_ghost_copy(OutPtrs u, int nf, const Gho
                                                     const GhostBox *__restrict__ boxes)
 {
     SGR_EXACT
-    const GhostBox bx = boxes[blockIdx.x];
+    const GhostBox bx = boxes[xcd_remap(blockIdx.x, gridDim.x)];
     const GhostPatch g = patches[bx.patch];
     const int ex = bx.e[0], ey = bx.e[1], n = ex * ey * bx.e[2];
     const uint64_t sy = g.sn0, sz = (uint64_t)g.sn0 * g.sn1;
