@@ -205,7 +205,7 @@ bool stencil_queue(uint64_t faces, uint64_t tiles)
 // and pointwise passes.
 bool one_pass(const sgr_params &p)
 {
-    return p.precision == SGR_PREC_FP64 && p.gauge == SGR_GAUGE_STANDARD && p.dissipation == SGR_DISS_KO;
+    return p.precision == SGR_PREC_FP64 && p.gauge == SGR_GAUGE_STANDARD;
 }
 
 // Do two arrays of `span` values share memory?
@@ -763,7 +763,7 @@ static hipError_t one_pass_chunks(sgr_plan *plan, LaunchArgs a, hipStream_t stre
     }
     if (e == hipSuccess && plan->pipe) e = hipEventRecord(plan->pev[1], plan->side);
     if (e == hipSuccess && plan->pipe) e = hipStreamWaitEvent(stream, plan->pev[1], 0);
-    for (int q = 1; q < 4 && e == hipSuccess && ev; q++) e = hipEventRecord(ev[q], stream);
+    for (int q = 1; q < (a.diss ? 2 : 4) && e == hipSuccess && ev; q++) e = hipEventRecord(ev[q], stream);
     return e;
 }
 
@@ -807,7 +807,9 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
     hipGetDevice(&cur);
     if (cur != plan->device) HIP_TRY(hipSetDevice(plan->device), "hipSetDevice");
     hipError_t e = a.diss ? launch_speeds(a, stream) : hipSuccess;  // once, over every node
-    if (a.fused && plan->lists.size() > 1) {
+    if (a.fused && a.diss) a.ev[2] = a.ev[3] = nullptr;  // they bracket k_tvb_add
+    if (e != hipSuccess) {
+    } else if (a.fused && plan->lists.size() > 1) {
         e = one_pass_chunks(plan, a, stream, ev);
     } else if (e == hipSuccess && plan->ntiles <= plan->chunk_tiles) {
         if (a.fused && plan->ntiles)
@@ -829,6 +831,11 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
         if (e == hipSuccess && ev) e = hipEventRecord(ev[1], stream);
         if (e == hipSuccess && ev) e = hipEventRecord(ev[2], stream);
         if (e == hipSuccess && ev) e = hipEventRecord(ev[3], stream);
+    }
+    if (e == hipSuccess && a.fused && a.diss) {
+        for (int q = 2; q < 4; q++) a.ev[q] = ev ? ev[q] : nullptr;
+        for (int k = 0; k < 2; k++) a.list[k] = plan->all[k];
+        e = launch_tvb(a, stream);
     }
     if (cur != plan->device) hipSetDevice(cur);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");

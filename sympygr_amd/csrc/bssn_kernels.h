@@ -81,4 +81,8 @@ hipError_t launch_rhs(const LaunchArgs &a, hipStream_t s);
 // TVB dissipation: the characteristic speeds at every node (before launch_rhs)
 hipError_t launch_speeds(const LaunchArgs &a, hipStream_t s);
 
+// and, after a one-pass call, the dissipation added to what it wrote (a two-pass
+// launch adds it to the tails itself)
+hipError_t launch_tvb(const LaunchArgs &a, hipStream_t s);
+
 }  // namespace sgr

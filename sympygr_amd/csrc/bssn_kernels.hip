@@ -695,7 +695,8 @@ __global__ __launch_bounds__(256) void k_speeds(FieldPtrs in, double *__restrict
 }
 
 // Adds sigma (D_x + D_y + D_z) of TVB3 or TVB5 to the tail of every field at
-// every interior point the launch's tiles own (after the stencil pass, which
+// every interior point the launch's tiles own (two-pass calls: mixed precision,
+// outputs over inputs; after the stencil pass, which
 // left the Kreiss-Oliger term out; the reference adds the dissipation after
 // the boundary conditions, rhs.cpp:766-802, so face points get it too).  Same
 // tile -> thread map as the pointwise kernel.

@@ -409,10 +409,11 @@ struct DescWords {
     }
 };
 
-// What one pass computes: the right-hand side of a system, or the constraints
+// What one pass computes: the right-hand side of a system, TVB dissipation added
+// to a finished right-hand side (or RK stage), or the constraints
 // (with Psi4): gt, chi -> Ricci without d Gt; K, Gt, At -> added to the sums as
 // they appear.
-enum class Pass { BSSN, CCZ4, CONSTRAINTS, PSI4 };
+enum class Pass { BSSN, CCZ4, TVB3, TVB5, CONSTRAINTS, PSI4 };
 
 // A pass's fields in the order they are processed (those with second
 // derivatives first) and where the table of their pointers holds which.
@@ -458,6 +459,14 @@ struct FieldTable {
     }
 };
 
+// TVB: the characteristic speeds along x, y, z (span nodes each) and the factor
+// of the dissipation.
+struct TvbArgs {
+    const double *lam;
+    uint64_t span;
+    double sigma;
+};
+
 // The tiles of one k_rhs launch: entries lo[x] .. lo[x + 1] - 1 of its list
 // belong to XCD x (workgroups go to the XCDs round-robin by id).
 struct TileRanges {
@@ -488,10 +497,11 @@ struct TileRanges {
 template <Pass PASS, bool UPWIND, bool GEN, bool RK, bool ROUND>
 __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out, const BlockDesc *__restrict__ blocks,
                                          const uint32_t *__restrict__ tile_block, const uint32_t *__restrict__ order,
-                                         const Params &P, const RkArgs &rk, const TileRanges &ranges)
+                                         const Params &P, const RkArgs &rk, const TileRanges &ranges,
+                                         const TvbArgs &tv = TvbArgs{})
 {
     typedef Fields<PASS> F;
-    constexpr bool MONITOR = F::MONITOR, CCZ4 = F::CCZ4;
+    constexpr bool MONITOR = F::MONITOR, CCZ4 = F::CCZ4, TVB5 = PASS == Pass::TVB5, TVB = TVB5 || PASS == Pass::TVB3;
     constexpr int NT = 512;
     constexpr int RS8 = 24, PS8 = RS8 * TH;       // 8^3: padded halo rows (conflict-free, see k_stencil)
     constexpr int USZ = GEN ? GEN_U_CAP : PS8 * TH;
@@ -499,9 +509,9 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
     constexpr int NPF = GEN ? 4 : 3;              // halo loads per thread, 16 bytes each
     constexpr int NB2 = GEN ? 1 : 2;              // buffers of DX and DY
     __shared__ __align__(16) double U[2 * USZ];
-    __shared__ double DX[NB2 * DXSZ];
-    __shared__ double DY[NB2 * DYSZ];
-    __shared__ double DB[MONITOR ? 1 : 9 * NT];   // each thread's d_j beta^i, at 3 i + j
+    __shared__ double DX[TVB ? 1 : NB2 * DXSZ];
+    __shared__ double DY[TVB ? 1 : NB2 * DYSZ];
+    __shared__ double DB[MONITOR || TVB ? 1 : 9 * NT];   // each thread's d_j beta^i, at 3 i + j
     __shared__ double SP[3];                      // sigma, lambda_2, 1 - lambda_3
 
     const int t = threadIdx.x;
@@ -541,7 +551,7 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
     }
     // (read from LDS where they are used: scalar loads of them were waited for
     // in every field, registers for them spilled)
-    if (!MONITOR && t == 0) SP[0] = P.ko_sigma, SP[1] = P.lambda[2], SP[2] = 1.0 - P.lambda[3];
+    if (!MONITOR && !TVB && t == 0) SP[0] = P.ko_sigma, SP[1] = P.lambda[2], SP[2] = 1.0 - P.lambda[3];
 
     // What the halo loads of one tile need.  A load takes two neighbours of a
     // row (16 bytes, 8-byte aligned), half as many instructions for the same
@@ -620,6 +630,7 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
         }
     };
     auto fetch_point = [&](const DescWords &D) __attribute__((always_inline)) {
+        if constexpr (TVB) return;
         int lx, ly, lz;
         bool has;
         point_of(thread(), D, lx, ly, lz, has);
@@ -1167,6 +1178,140 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
 #undef SGR_K
     };
 
+    // One tile of TVB dissipation (tvb in stencils.h states the forms), added to
+    // the outputs.  An axis is pre (W0 X0 - W1 X1 + W2 X2 - ...): the weights W,
+    // speeds times coefficients, are the same for every field; X are differences
+    // of neighbours (TVB5) or values (TVB3, one-sided forms).  EDGE: a tile with
+    // points of the one-sided forms or at a flagged face.
+    auto tvb_tile = [&](auto edge_, const DescWords &D, const TileCoord &tc, const ConstBlock B, uint32_t mnext,
+                        uint32_t &next, uint32_t &nnext, DescWords &Dnext, TileCoord &tnc) __attribute__((always_inline)) {
+        SGR_EXACT
+        constexpr bool EDGE = decltype(edge_)::value;
+        constexpr int NW = TVB5 ? 6 : 5;
+        const int TX = GEN ? D.tdim(0) : T, TY = GEN ? D.tdim(1) : T, TZ = GEN ? D.tdim(2) : T;
+        const int HX = TX + 2 * GW, HY = TY + 2 * GW, td[3] = {TX, TY, TZ};
+        const int ls[3] = {1, GEN ? HX : RS8, GEN ? HX * HY : PS8};  // strides in U
+        const int nn[3] = {D.n(0), D.n(1), D.n(2)}, st[3] = {1, nn[0], nn[0] * nn[1]};
+        const uint32_t bflag = D.bflag();
+        const uint64_t obase = D.offset();
+        int lp[3];
+        bool own;
+        point_of(thread(), D, lp[0], lp[1], lp[2], own);
+        const int pos[3] = {tc.i0 + lp[0], tc.j0 + lp[1], tc.k0 + lp[2]};
+        own = own && pos[0] >= tc.oi && pos[1] >= tc.oj && pos[2] >= tc.ok;
+        const int gp = pos[0] + nn[0] * (pos[1] + nn[1] * pos[2]);
+        const int uc = (lp[0] + GW) * ls[0] + (lp[1] + GW) * ls[1] + (lp[2] + GW) * ls[2];
+        double W[3][NW], pre[3];
+        bool clo[3], chi_[3];                 // the tile reaches the closures of a flagged face (uniform)
+        bool face[3];                         // point of a Kreiss-Oliger closure
+        bool head[3], tail[3];                // point of a one-sided form
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const int o = d == 0 ? tc.i0 : d == 1 ? tc.j0 : tc.k0;
+            clo[d] = EDGE && (bflag >> (2 * d) & 1u) && o < GW + 3;
+            chi_[d] = EDGE && (bflag >> (2 * d + 1) & 1u) && o + td[d] - 1 >= nn[d] - GW - 3;
+            face[d] = (clo[d] && pos[d] < GW + 3) || (chi_[d] && pos[d] >= nn[d] - GW - 3);
+            head[d] = EDGE && TVB5 && !face[d] && pos[d] == GW;
+            tail[d] = EDGE && TVB5 && !face[d] && !head[d] && pos[d] == nn[d] - GW - 1;
+            pre[d] = TVB5 ? (d == 2 ? B->ax[2].ko_pre : 2.0 / 75.0 / B->ax[d].h) : -1.0 / 12.0 / B->ax[d].h;
+            if (EDGE && TVB5) pre[d] = head[d] || tail[d] ? 1.0 / B->ax[d].smr1 : pre[d];
+            const SGR_GLOBAL double *l = (const SGR_GLOBAL double *)(uint64_t)(tv.lam + d * tv.span + obase) + gp;
+            const int s = st[d];
+            if constexpr (!TVB5) {
+                W[d][0] = l[-2 * s], W[d][1] = 4.0 * l[-s], W[d][2] = 6.0 * l[0], W[d][3] = 4.0 * l[s], W[d][4] = l[2 * s];
+            } else {
+                const double l3 = l[tail[d] ? -4 * s : 3 * s], l2 = l[2 * s], l1 = l[s], l0 = l[0];
+                const double m1 = l[-s], m2 = l[-2 * s], m3 = l[-3 * s];
+                W[d][0] = larger(l3, l2), W[d][1] = 5.0 * larger(l2, l1), W[d][2] = 10.0 * larger(l1, l0);
+                W[d][3] = 10.0 * larger(l0, m1), W[d][4] = 5.0 * larger(m1, m2), W[d][5] = larger(m2, m3);
+                if (head[d])
+                    W[d][0] = l3, W[d][1] = 6.0 * l2, W[d][2] = 15.0 * l1, W[d][3] = 19.0 * l0, W[d][4] = 12.0 * m1,
+                    W[d][5] = 3.0 * m2;
+                if (tail[d])
+                    W[d][0] = l3, W[d][1] = 6.0 * m3, W[d][2] = 15.0 * m2, W[d][3] = 19.0 * m1, W[d][4] = 12.0 * l0,
+                    W[d][5] = 3.0 * l1;
+            }
+        }
+        // what is added to: loaded a field ahead, like the halo tile (waited for in
+        // its own field, a load waits for the store of the field before as well)
+        double av = 0.0, nv = 0.0;
+        auto ahead = [&](int p) __attribute__((always_inline)) {
+            if (!RK || rk.stage < 3) av = (tout.get(p) + obase)[gp];
+            if (RK) nv = (tnext.get(p) + obase)[gp];
+        };
+        ahead(0);
+        auto field = [&](auto last_, int p) __attribute__((always_inline)) {
+            SGR_EXACT
+            SGR_GLOBAL double *o = tout.get(p) + obase, *nx = RK ? tnext.get(p) + obase : o;
+            const double *c = &U[b * USZ + uc];
+            const double c0 = c[0];
+            uint64_t bp = (uint64_t)B;  // (as in run_tile)
+            asm volatile("" : "+s"(bp));
+            double Dd[3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const int s = ls[d];
+                if constexpr (!TVB5) {
+                    Dd[d] = pre[d] * (W[d][0] * c[-2 * s] - W[d][1] * c[-s] + W[d][2] * c0 - W[d][3] * c[s] + W[d][4] * c[2 * s]);
+                } else {
+                    double v[7], X[6];
+                    // (the one-sided form at the end reads four back: inside the halo,
+                    // no tile extent is 1 and the last point is the tile's last)
+                    v[0] = c[tail[d] ? -4 * s : 3 * s];
+                    v[1] = c[2 * s], v[2] = c[s], v[3] = c0, v[4] = c[-s], v[5] = c[-2 * s], v[6] = c[-3 * s];
+#pragma unroll
+                    for (int k = 0; k < 6; k++) {
+                        X[k] = v[k] - v[k + 1];
+                        if constexpr (EDGE) {
+                            X[k] = head[d] ? v[k] : X[k];
+                            X[k] = tail[d] ? v[k == 0 ? 0 : 7 - k] : X[k];
+                        }
+                    }
+                    Dd[d] = pre[d] * (W[d][0] * X[0] - W[d][1] * X[1] + W[d][2] * X[2] - W[d][3] * X[3] + W[d][4] * X[4] -
+                                      W[d][5] * X[5]);
+                }
+                if (EDGE && (clo[d] || chi_[d])) {
+                    double t9[9];
+                    face_taps(c, s, pos[d], nn[d], clo[d], chi_[d], t9);
+                    const double k = ko_face(t9, pos[d], nn[d], clo[d], chi_[d], axis_of((ConstBlock)bp, d));
+                    Dd[d] = face[d] ? k : Dd[d];
+                }
+            }
+            const double a = tv.sigma * ((Dd[0] + Dd[1]) + Dd[2]);
+            put(&U[(1 - b) * USZ]);
+            double s0 = av + (RK ? rk.w * a : a), s1 = nv + (RK && rk.stage < 3 ? rk.cn * a : rk.w * a);
+            asm volatile("" : "+v"(s0), "+v"(s1));  // (formed before the next loads are issued)
+            __syncthreads();
+            if (p + 1 < F::N) ahead(p + 1);
+            if constexpr (!decltype(last_)::value) {
+                keep_dst();
+                fetch(p + 2 < F::N ? p + 2 : 0);
+            }
+            if (own) {
+                if (!RK || rk.stage < 3) o[gp] = s0;
+                if (RK) nx[gp] = s1;
+            }
+            b ^= 1;
+        };
+        const auto yes = std::true_type{};
+        const auto no = std::false_type{};
+        uint32_t word = tile_of(mnext);
+#pragma unroll 1
+        for (int p = 0; p < 6; p++) field(no, p);
+        next = first(word);
+        word = block_of(next);
+#pragma unroll 1
+        for (int p = 6; p < 12; p++) field(no, p);
+        nnext = first(word);
+        Dnext.load(blocks + nnext, thread() & 63);
+#pragma unroll 1
+        for (int p = 12; p < F::N - 2; p++) field(no, p);
+        tnc = Dnext.coord(next);
+        aim(Dnext, tnc);
+        field(no, F::N - 2);
+        field(yes, F::N - 1);
+    };
+
     uint32_t tile = first(tile_of(m)), nb = first(block_of(tile));
     DescWords D;
     D.load(blocks + nb, t & 63);
@@ -1188,13 +1333,19 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
             const int o = d == 0 ? tc.i0 : d == 1 ? tc.j0 : tc.k0;
             face |= ((D.bflag() >> (2 * d)) & 1u && o < GW + 3) ||
                     ((D.bflag() >> (2 * d + 1)) & 1u && o + (GEN ? D.tdim(d) : T) - 1 >= D.n(d) - GW - 3);
+            if (TVB5) face |= o == GW || o + (GEN ? D.tdim(d) : T) >= D.n(d) - GW;  // one-sided forms
         }
         uint32_t next = 0, nnext = 0;
         DescWords Dnext;
         TileCoord tnc;
         const ConstBlock B = (ConstBlock)(uint64_t)(blocks + first(nb));
-        if (face) run_tile(std::true_type{}, D, tc, B, mnext, next, nnext, Dnext, tnc);
-        else run_tile(std::false_type{}, D, tc, B, mnext, next, nnext, Dnext, tnc);
+        if constexpr (TVB) {
+            if (face) tvb_tile(std::true_type{}, D, tc, B, mnext, next, nnext, Dnext, tnc);
+            else tvb_tile(std::false_type{}, D, tc, B, mnext, next, nnext, Dnext, tnc);
+        } else {
+            if (face) run_tile(std::true_type{}, D, tc, B, mnext, next, nnext, Dnext, tnc);
+            else run_tile(std::false_type{}, D, tc, B, mnext, next, nnext, Dnext, tnc);
+        }
         if (m >= end) break;
         tile = next, nb = nnext, D = Dnext, tc = tnc;
     }

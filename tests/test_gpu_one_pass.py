@@ -139,3 +139,38 @@ def test_ccz4_edge_sizes_against_oracle(n, bflag, adv):
     for a, w in ((nxt, 0.5 * dt), (acc, dt / 6.0)):
         assert (np.abs(of(a.cpu()) - (u0 + w * got)) <= 2 * eps * (np.abs(u0) + np.abs(w * got))).all()
     assert (out.cpu().reshape(25, s[2], s[1], s[0])[:, :3] == 5.0).all()
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("diss,bflag", [("tvb3", 0), ("tvb5", 0), ("tvb3", 63), ("tvb5", 63), ("tvb5", 38)])
+def test_tvb_edge_sizes_against_oracle(n, diss, bflag):
+    """TVB dissipation, added by a pass of its own over the same tiles (one-sided
+    forms at the first and last point, closures at flagged faces), same sizes
+    and bar; the second and the last RK stage from it, to a rounding of each
+    of their terms."""
+    import pyoracle as po
+    import torch
+    import sympygr_amd as sgr
+    bl, u = _block(n, bflag, 9 + n[1])
+    plan = sgr.Plan(bl, sgr.params(adv="upwind", ko_sigma=0.1, dissipation=diss))
+    du = torch.from_numpy(u).cuda()
+    out = torch.full_like(du, 5.0)
+    plan.rhs(out, du)
+    base, dt = torch.full_like(du, 0.25), 0.0625
+    acc, nxt, end = base.clone(), torch.full_like(du, 5.0), torch.full_like(du, 5.0)
+    plan.rk4_stage(1, dt, base, du, acc, nxt)
+    plan.rk4_stage(3, dt, base, du, base, end)
+    torch.cuda.synchronize()
+    s = bl.sz[0]
+    ref = po.rhs_block(u, s, bl.pmin[0], bl.pmax[0], bflag, po.make_params(upwind=True, ko_sigma=0.1, dissipation=diss))
+    got = interior(out.cpu().numpy(), s)
+    assert normwise(got, interior(ref, s)).max() <= 1e-12
+    eps = 2.0 ** -52
+    for a, w in ((acc, dt / 3.0), (nxt, dt / 2.0), (end, dt / 6.0)):
+        a = interior(a.cpu().numpy(), s)
+        # the right-hand side and the dissipation are added one after the other
+        scale = 0.25 + np.abs(w * got).max(axis=(1, 2, 3), keepdims=True)
+        assert (np.abs(a - (0.25 + w * got)) <= 4 * eps * scale).all()
+    for a in (out, nxt, end):
+        a = a.cpu().numpy().reshape(24, s[2], s[1], s[0])
+        assert (a[:, :3] == 5.0).all() and (a[:, :, :, -3:] == 5.0).all()
