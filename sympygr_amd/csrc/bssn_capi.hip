@@ -232,43 +232,54 @@ bool one_pass_call(const sgr_params &p, const FieldPtrs &in, const OutPtrs &out,
     return true;
 }
 
-// Does RHS tile lt of block d come within three points of a flagged face
-// (where k_rhs takes the closure forms)?
-bool closure_tile(const BlockDesc &d, uint32_t lt)
+// Which RHS tiles come within three points of a flagged face (where k_rhs takes
+// the closure forms), by tile number.
+std::vector<uint8_t> closure_tiles(const std::vector<BlockDesc> &hb, const std::vector<uint32_t> &tile_block)
 {
-    const int t[3] = {(int)(lt % d.ntile[0]), (int)(lt / d.ntile[0] % d.ntile[1]), (int)(lt / (d.ntile[0] * d.ntile[1]))};
-    for (int k = 0; k < 3; k++) {
-        const int o = std::min(GW + d.tdim[k] * t[k], d.n[k] - GW - d.tdim[k]);
-        if ((d.bflag >> (2 * k) & 1u && o < GW + 3) ||
-            (d.bflag >> (2 * k + 1) & 1u && o + d.tdim[k] - 1 >= d.n[k] - GW - 3))
-            return true;
+    std::vector<uint8_t> slow(tile_block.size(), 0);
+    std::vector<uint8_t> near[3];
+    for (size_t i = 0; i < tile_block.size();) {
+        const BlockDesc &d = hb[tile_block[i]];
+        const size_t n = (size_t)d.ntile[0] * d.ntile[1] * d.ntile[2];
+        if (d.bflag) {
+            for (int k = 0; k < 3; k++) {
+                near[k].assign(d.ntile[k], 0);
+                for (int t = 0; t < d.ntile[k]; t++) {
+                    const int o = std::min(GW + d.tdim[k] * t, d.n[k] - GW - d.tdim[k]);
+                    near[k][t] = (d.bflag >> (2 * k) & 1u && o < GW + 3) ||
+                                 (d.bflag >> (2 * k + 1) & 1u && o + d.tdim[k] - 1 >= d.n[k] - GW - 3);
+                }
+            }
+            uint8_t *q = &slow[i];
+            for (int z = 0; z < d.ntile[2]; z++)
+                for (int y = 0; y < d.ntile[1]; y++)
+                    for (int x = 0; x < d.ntile[0]; x++) *q++ = near[0][x] | near[1][y] | near[2][z];
+        }
+        i += n;
     }
-    return false;
+    return slow;
 }
 
 // The list of one k_rhs launch over tiles t0 .. t0 + n - 1: eight consecutive
 // ranges of about equal cost (CLOSURE_COST: measured ratio of the two kinds of
 // tiles), in each the tiles without closure forms first.  Appends to `order`.
 constexpr double CLOSURE_COST = 1.9;
-TileList tile_list(const std::vector<BlockDesc> &hb, const std::vector<uint32_t> &tile_block, uint32_t t0, uint32_t n,
-                   std::vector<uint32_t> &order)
+TileList tile_list(const std::vector<uint8_t> &slow, uint32_t t0, uint32_t n, std::vector<uint32_t> &order)
 {
     TileList l{};
-    std::vector<bool> slow(n);
-    double total = 0.0, seen = 0.0;
-    for (uint32_t i = 0; i < n; i++) {
-        const BlockDesc &d = hb[tile_block[t0 + i]];
-        slow[i] = d.bflag && closure_tile(d, t0 + i - d.tile_base);
-        total += slow[i] ? CLOSURE_COST : 1.0;
-    }
+    uint64_t nslow = 0;
+    for (uint32_t i = 0; i < n; i++) nslow += slow[t0 + i];
+    const double total = n + (CLOSURE_COST - 1.0) * nslow;
+    double seen = 0.0;
     uint32_t i = 0;
     for (int x = 0; x < 8; x++) {
         l.lo[x] = (uint32_t)order.size();
         const uint32_t i0 = i;
-        for (; i < n && (x == 7 || seen < total * (x + 1) / 8); i++) seen += slow[i] ? CLOSURE_COST : 1.0;
-        for (int pass = 0; pass < 2; pass++)
+        const double until = x == 7 ? HUGE_VAL : total * (x + 1) / 8;
+        for (; i < n && seen < until; i++) seen += slow[t0 + i] ? CLOSURE_COST : 1.0;
+        for (uint8_t pass = 0; pass < 2; pass++)
             for (uint32_t k = i0; k < i; k++)
-                if (slow[k] == (pass == 1)) order.push_back(t0 + k);
+                if (slow[t0 + k] == pass) order.push_back(t0 + k);
     }
     l.lo[8] = (uint32_t)order.size();
     return l;
@@ -581,9 +592,11 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
     }
     p->ntiles = (uint32_t)tile_block.size();
     std::vector<uint32_t> order;
+    const std::vector<uint8_t> slow = closure_tiles(p->hblocks, tile_block);
     if (p->ntiles) {
-        p->all[0] = tile_list(p->hblocks, tile_block, 0, p->nfast, order);
-        p->all[1] = tile_list(p->hblocks, tile_block, p->nfast, p->ntiles - p->nfast, order);
+        order.reserve(2 * (size_t)p->ntiles);
+        p->all[0] = tile_list(slow, 0, p->nfast, order);
+        p->all[1] = tile_list(slow, p->nfast, p->ntiles - p->nfast, order);
     }
     if (one_pass(*params) && p->ntiles) {
         const uint64_t nc = (p->ntiles + p->chunk_tiles - 1) / p->chunk_tiles;
@@ -593,7 +606,7 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
             for (int k = 0; k < 2; k++) {
                 const uint64_t k0 = k ? p->nfast : 0, n = k ? p->ntiles - p->nfast : p->nfast;
                 const uint64_t a = n * c / nc, e = n * (c + 1) / nc;
-                l[k] = tile_list(p->hblocks, tile_block, (uint32_t)(k0 + a), (uint32_t)(e - a), order);
+                l[k] = tile_list(slow, (uint32_t)(k0 + a), (uint32_t)(e - a), order);
             }
             p->lists.push_back(l);
         }
