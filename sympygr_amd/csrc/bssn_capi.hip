@@ -90,9 +90,52 @@ const TileShapeEntry kTileTable[] = {
     {{0, 0, 0}, {T, T, T}},
 };
 
+// The tile shape the one-pass kernels take for n[0] x n[1] x n[2] interior
+// points.  A tile holds a CU for its whole run whatever it covers: 47-51 us for
+// 8^3 (constant strides, no second barrier), 66-71 us for another shape, nearly
+// the same for 125 points as for 500.  So the shape with the fewest tiles,
+// weighted with that ratio, of equal ones the one with the smallest halo: 10^3
+// as two 10 x 10 x 5 tiles instead of eight 8^3: 13^3 blocks of it take 1.25
+// instead of 3.23 ms; 12^3 points 2.02 -> 1.38 ms, 18^3 1.74 -> 1.14 ms.
+// few: all the launch's 8^3 tiles run at once, then the time of one tile counts
+// (one block of 25^3 points as 64 8^3 tiles 160 us, as 18 larger ones 178 us).
+constexpr double GENERAL_TILE_COST = 1.4;
+constexpr uint64_t FEW_TILES = 256;  // a workgroup on every CU
+uint64_t cube_tiles(const sgr_block &b)
+{
+    uint64_t t = 1;
+    for (int k = 0; k < 3; k++) t *= (b.sz[k] - 6 + T - 1) / T;
+    return t;
+}
+void one_pass_shape(const int n[3], bool few, int td[3])
+{
+    auto pieces = [&](int k, int x) { return (double)((n[k] + x - 1) / x); };
+    auto is_cube = [&]() { return td[0] == T && td[1] == T && td[2] == T; };
+    for (int k = 0; k < 3; k++) td[k] = std::min(T, n[k]);
+    if (few) return;
+    double best = (is_cube() ? 1.0 : GENERAL_TILE_COST) * pieces(0, T) * pieces(1, T) * pieces(2, T);
+    int halo = (td[0] + 2 * GW) * (td[1] + 2 * GW) * (td[2] + 2 * GW);
+    std::vector<int> e[3];  // extents that split an axis evenly
+    for (int k = 0; k < 3; k++)
+        for (int p = 1; p <= n[k] / 2; p++) {
+            const int x = (n[k] + p - 1) / p;
+            if (x <= TILE_PTS / 4 && (e[k].empty() || e[k].back() != x)) e[k].push_back(x);
+        }
+    for (int x : e[0])
+        for (int y : e[1])
+            for (int z : e[2]) {
+                if (!tile_shape_ok(x, y, z) || (x == T && y == T && z == T)) continue;
+                const double c = GENERAL_TILE_COST * pieces(0, x) * pieces(1, y) * pieces(2, z);
+                const int h = (x + 2 * GW) * (y + 2 * GW) * (z + 2 * GW);
+                if (c > best || (c == best && (h >= halo || is_cube()))) continue;
+                best = c, halo = h, td[0] = x, td[1] = y, td[2] = z;
+            }
+}
+
 // The RHS tile shape of a block: SGR_TILE_SHAPE=tx,ty,tz (every block; for
-// tuning and tests), else the table, else 8^3.
-int tile_shape(const sgr_block &b, int td[3])
+// tuning and tests), else for the one-pass kernels the rule above, for the two
+// passes the table or 8^3.
+int tile_shape(const sgr_block &b, bool one_pass, bool few, int td[3])
 {
     td[0] = td[1] = td[2] = T;
     if (const char *sv = getenv("SGR_TILE_SHAPE")) {
@@ -101,6 +144,9 @@ int tile_shape(const sgr_block &b, int td[3])
             return fail(SGR_E_INVALID, std::string("SGR_TILE_SHAPE=") + sv +
                                            " is not a tile shape (tx,ty,tz >= 2, at most 512 points, within the "
                                            "stencil kernel's LDS arrays)");
+    } else if (one_pass) {
+        const int n[3] = {(int)b.sz[0] - 6, (int)b.sz[1] - 6, (int)b.sz[2] - 6};
+        one_pass_shape(n, few, td);
     } else {
         for (const TileShapeEntry &e : kTileTable) {
             if (e.n[0] == b.sz[0] - 6 && e.n[1] == b.sz[1] - 6 && e.n[2] == b.sz[2] - 6) {
@@ -505,9 +551,20 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
     // tiles (8^3) in block order
     std::vector<uint32_t> tile_block, tile_block8;
     std::vector<int> shape(3 * (size_t)nblocks);
+    uint64_t cubes = 0;
     for (uint32_t b = 0; b < nblocks; b++) {
         rc = validate_block(blocks[b], b);
-        if (!rc) rc = tile_shape(blocks[b], &shape[3 * b]);
+        if (rc) {
+            delete p;
+            return rc;
+        }
+        cubes += cube_tiles(blocks[b]);
+    }
+    std::map<std::array<uint32_t, 3>, uint32_t> first;  // the first block of a size
+    for (uint32_t b = 0; b < nblocks; b++) {
+        const auto like = first.insert({{blocks[b].sz[0], blocks[b].sz[1], blocks[b].sz[2]}, b}).first->second;
+        if (like == b) rc = tile_shape(blocks[b], one_pass(*params), cubes <= FEW_TILES, &shape[3 * b]);
+        else std::copy_n(&shape[3 * like], 3, &shape[3 * b]);
         if (rc) {
             delete p;
             return rc;
@@ -1365,10 +1422,10 @@ int sgr_rhs_block_noalloc(double *const out[SGR_NUM_VARS], const double *const i
     for (int f = 0; f < nf; f++)
         if (!in[f] || !out[f]) return fail(SGR_E_INVALID, "null field pointer");
     int td[3];
-    rc = tile_shape(b, td);
+    rc = tile_shape(b, false, false, td);
     if (rc) return rc;
-    const BlockDesc d = block_desc(b, td, 0, 0);
-    const uint64_t ntiles = (uint64_t)d.ntile[0] * d.ntile[1] * d.ntile[2];
+    BlockDesc d = block_desc(b, td, 0, 0);
+    uint64_t ntiles = (uint64_t)d.ntile[0] * d.ntile[1] * d.ntile[2];
     const size_t wsz = params->precision == SGR_PREC_MIXED ? sizeof(float) : sizeof(double);
     const uint64_t need = NOALLOC_WS_OFF + ntiles * rhs_tile_bytes(wsz, nf);
     if (ntiles > NOALLOC_MAX_TILES || need > NOALLOC_SCRATCH_BYTES) {
@@ -1377,6 +1434,20 @@ int sgr_rhs_block_noalloc(double *const out[SGR_NUM_VARS], const double *const i
                  "block of %llu tiles needs %.1f MiB of scratch; the allocation-free entry holds %llu MiB",
                  (unsigned long long)ntiles, need / 1048576.0, (unsigned long long)(NOALLOC_SCRATCH_BYTES >> 20));
         return fail(SGR_E_INVALID, msg);
+    }
+    LaunchArgs a{};
+    for (int f = 0; f < nf; f++) {
+        a.in.p[f] = in[f];
+        a.out.p[f] = out[f];
+    }
+    a.rk.stage = -1;
+    a.fused = one_pass_call(*params, a.in, a.out, a.rk, offset + (uint64_t)sz[0] * sz[1] * sz[2]);
+    if (a.fused) {  // (needs the map of its tiles only; the refusal above stays that of the two passes)
+        rc = tile_shape(b, true, cube_tiles(b) <= FEW_TILES, td);
+        if (rc) return rc;
+        d = block_desc(b, td, 0, 0);
+        ntiles = (uint64_t)d.ntile[0] * d.ntile[1] * d.ntile[2];
+        if (ntiles > NOALLOC_MAX_TILES) return fail(SGR_E_INVALID, "too many tiles");
     }
     int device = 0;
     HIP_TRY(hipGetDevice(&device), "hipGetDevice");
@@ -1387,11 +1458,6 @@ int sgr_rhs_block_noalloc(double *const out[SGR_NUM_VARS], const double *const i
     uint32_t *d_map = (uint32_t *)(sp + NOALLOC_MAP_OFF);
     hipLaunchKernelGGL(k_setup_block, dim3(1), dim3(256), 0, stream, d, d_desc, d_map, (uint32_t)ntiles);
     HIP_TRY(hipGetLastError(), "k_setup_block launch");
-    LaunchArgs a{};
-    for (int f = 0; f < nf; f++) {
-        a.in.p[f] = in[f];
-        a.out.p[f] = out[f];
-    }
     a.blocks = d_desc;
     a.tile_block = d_map;
     a.ntiles = (uint32_t)ntiles;
@@ -1404,8 +1470,6 @@ int sgr_rhs_block_noalloc(double *const out[SGR_NUM_VARS], const double *const i
     a.upwind = params->adv_mode == SGR_ADV_UPWIND;
     a.mixed = params->precision == SGR_PREC_MIXED;
     a.ccz4 = nf == NF_CCZ4;
-    a.rk.stage = -1;
-    a.fused = one_pass_call(*params, a.in, a.out, a.rk, offset + (uint64_t)sz[0] * sz[1] * sz[2]);
     for (int x = 0; x < 9; x++) a.list[is_cube8(d) ? 0 : 1].lo[x] = (uint32_t)(ntiles * x / 8);
     const hipError_t e = launch_rhs(a, stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");

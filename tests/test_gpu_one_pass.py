@@ -174,3 +174,31 @@ def test_tvb_edge_sizes_against_oracle(n, diss, bflag):
     for a in (out, nxt, end):
         a = a.cpu().numpy().reshape(24, s[2], s[1], s[0])
         assert (a[:, :3] == 5.0).all() and (a[:, :, :, -3:] == 5.0).all()
+
+
+@pytest.mark.parametrize("sizes", [(9, 9, 9), (10, 10, 10), (11, 12, 12), (18, 20, 9), (26, 27, 7), (7, 33, 12)])
+def test_shapes_chosen_by_the_tile_count(sizes):
+    """Enough blocks that the rule picks larger tiles than 8^3 (a block by itself
+    takes 8^3): fewer tiles than 8^3 would make, and the same bits."""
+    import torch
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    bl = data.BlockList()
+    cubes = 1
+    for k in sizes:
+        cubes *= -(-k // 8)
+    count = 256 // cubes + 5
+    for b in range(count):
+        lo = (-1.0 + 0.02 * b, -0.5, -0.7)
+        sz = tuple(k + 6 for k in sizes)
+        bl.add(sz, lo, tuple(p + 0.04 * (s - 1) for p, s in zip(lo, sz)), (b * 11) & 63)
+    u = data.fill_blocks(bl, backend="torch", device="cuda", kind="perturbed", seed=5, amp=1e-2, lo=-1.0, L=2.0)
+    prm = sgr.params(adv="upwind", ko_sigma=0.1)
+    out, ref = torch.full_like(u, 5.0), torch.full_like(u, 5.0)
+    plan = sgr.Plan(bl, prm)
+    assert plan.info().tiles < cubes * count
+    plan.rhs(out, u)
+    for b in range(count):
+        sgr.rhs_block(ref, u, bl.offsets[b], bl.pmin[b], bl.pmax[b], bl.sz[b], bl.bflag[b], prm)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
