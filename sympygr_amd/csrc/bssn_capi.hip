@@ -92,14 +92,14 @@ const TileShapeEntry kTileTable[] = {
 
 // The tile shape the one-pass kernels take for n[0] x n[1] x n[2] interior
 // points.  A tile holds a CU for its whole run whatever it covers: 47-51 us for
-// 8^3 (constant strides, no second barrier), 66-71 us for another shape, nearly
-// the same for 125 points as for 500.  So the shape with the fewest tiles,
-// weighted with that ratio, of equal ones the one with the smallest halo: 10^3
-// as two 10 x 10 x 5 tiles instead of eight 8^3: 13^3 blocks of it take 1.25
-// instead of 3.23 ms; 12^3 points 2.02 -> 1.38 ms, 18^3 1.74 -> 1.14 ms.
+// 8^3 (constant strides), 63-69 us for another shape, nearly the same for 125
+// points as for 500.  So the shape with the fewest tiles, weighted with that
+// ratio, of equal ones the one with the smallest halo: 10^3 as two 10 x 10 x 5
+// tiles instead of eight 8^3 (13^3 such blocks: 3.23 -> 1.19 ms; 11^3 blocks of
+// 12^3 points 2.02 -> 1.31 ms, 7^3 of 18^3 1.74 -> 1.08 ms).
 // few: all the launch's 8^3 tiles run at once, then the time of one tile counts
 // (one block of 25^3 points as 64 8^3 tiles 160 us, as 18 larger ones 178 us).
-constexpr double GENERAL_TILE_COST = 1.4;
+constexpr double GENERAL_TILE_COST = 1.35;
 constexpr uint64_t FEW_TILES = 256;  // a workgroup on every CU
 uint64_t cube_tiles(const sgr_block &b)
 {

@@ -482,7 +482,8 @@ struct TileRanges {
 //   DB  the thread's first derivatives of the shift, parked
 // With both double-buffered a field takes one barrier: stencils and the stores
 // of DX, DY and the next U before it, mixed derivatives and algebra after it.
-// The general shapes have room for one DX and DY and take a second barrier.
+// General shapes of a large halo have room for one DX and DY and take a second
+// barrier.
 // The grid is persistent: a workgroup takes every (gridDim.x / 8)-th tile of
 // its XCD's range, and the next tile's first fields and point values are
 // fetched during the last fields of the current one.  Tiles that reach a
@@ -505,12 +506,12 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
     constexpr int NT = 512;
     constexpr int RS8 = 24, PS8 = RS8 * TH;       // 8^3: padded halo rows (conflict-free, see k_stencil)
     constexpr int USZ = GEN ? GEN_U_CAP : PS8 * TH;
-    constexpr int DXSZ = GEN ? GEN_DX_CAP : T * TH * TH, DYSZ = GEN ? GEN_DY_CAP : T * T * TH;
+    constexpr int DXSZ = T * TH * TH, DYSZ = T * T * TH;
+    constexpr int DCAP = 4478;                    // general shapes: one buffer of D_x and D_y, what LDS has left
     constexpr int NPF = GEN ? 4 : 3;              // halo loads per thread, 16 bytes each
-    constexpr int NB2 = GEN ? 1 : 2;              // buffers of DX and DY
     __shared__ __align__(16) double U[2 * USZ];
-    __shared__ double DX[TVB ? 1 : NB2 * DXSZ];
-    __shared__ double DY[TVB ? 1 : NB2 * DYSZ];
+    __shared__ double DX[TVB ? 1 : GEN ? 2 * DCAP : 2 * DXSZ];  // general shapes: DY behind DX
+    __shared__ double DY[TVB || GEN ? 1 : 2 * DYSZ];
     __shared__ double DB[MONITOR || TVB ? 1 : 9 * NT];   // each thread's d_j beta^i, at 3 i + j
     __shared__ double SP[3];                      // sigma, lambda_2, 1 - lambda_3
 
@@ -655,7 +656,8 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
         const int TX = GEN ? D.tdim(0) : T, TY = GEN ? D.tdim(1) : T, TZ = GEN ? D.tdim(2) : T;
         const int HX = TX + 2 * GW, HY = TY + 2 * GW;
         const int RS = GEN ? HX : RS8, PS = GEN ? HX * HY : PS8;
-        const int DXZ = TX * HY, DYZ = TX * TY;
+        const int DXZ = TX * HY, DYZ = TX * TY, dy0 = DXZ * (TZ + 2 * GW);
+        const bool two = !GEN || dy0 + DYZ * (TZ + 2 * GW) <= DCAP;  // do two of the buffers fit?
         const int n0 = D.n(0), n1 = D.n(1), n2 = D.n(2);
         const uint32_t bflag = D.bflag();
         const bool lo0 = FACE && (bflag & 1u), hi0 = FACE && (bflag & 2u), lo1 = FACE && (bflag & 4u);
@@ -714,7 +716,7 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
             const int uc = (lx + GW) + RS * (ly + GW) + PS * (lz + GW);
             const int cx = lx + TX * (ly + GW) + DXZ * (lz + GW), cy = lx + TX * ly + DYZ * (lz + GW);
             const double *c = &U[b * USZ + uc];
-            double *dx = &DX[(NB2 - 1) * b * DXSZ], *dy = &DY[(NB2 - 1) * b * DYSZ];
+            double *dx = &DX[GEN ? (two ? b * DCAP : 0) : b * DXSZ], *dy = GEN ? dx + dy0 : &DY[b * DYSZ];
             // the block's constants, read again in every field: fewer scalar
             // registers held across it
             uint64_t bp = (uint64_t)B;
@@ -829,7 +831,7 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
                 h[1] = d1_tile(cxp, TX, pj, n1, clo1, chi1, a1);   // D_y D_x
                 h[2] = d1_tile(cxp, DXZ, pk, n2, clo2, chi2, a2);  // D_z D_x
                 h[4] = d1_tile(cyp, DYZ, pk, n2, clo2, chi2, a2);  // D_z D_y
-                if (NB2 == 1) __syncthreads();  // DX and DY are read
+                if (!two) __syncthreads();  // DX and DY are read
             }
             if constexpr (ROUND) {
 #pragma unroll
