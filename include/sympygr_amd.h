@@ -151,12 +151,12 @@ int sgr_rhs(sgr_plan *plan, double *const out[SGR_NUM_VARS], const double *const
 
 /* Same as sgr_rhs, and records events[0..1] around the stencil pass and
  * events[2..3] around the pointwise kernel on `stream` (hipEventElapsedTime
- * then gives each pass's duration).  A one-pass plan (FP64, BSSN, standard
- * gauge, Kreiss-Oliger) has one kernel: events[0..1] bracket it, events[2..3]
- * are recorded after it.  For a plan that runs in several
- * workspace chunks (pipelined or not), events[0..1] bracket the whole call
- * and events[2..3] are recorded at its end.  No reference counterpart: it
- * exists for measurement. */
+ * then gives each pass's duration).  A one-pass plan (FP64, standard gauge)
+ * has one kernel: events[0..1] bracket it, events[2..3] are recorded after it
+ * (with TVB dissipation they bracket the pass that adds it).  For a plan that
+ * runs in several workspace chunks (pipelined or not), events[0..1] bracket
+ * the whole call (without that pass) and events[2..3] are recorded at its
+ * end.  No reference counterpart: it exists for measurement. */
 int sgr_rhs_events(sgr_plan *plan, double *const out[SGR_NUM_VARS], const double *const in[SGR_NUM_VARS],
                    hipStream_t stream, hipEvent_t events[4]);
 

@@ -1,4 +1,4 @@
-"""Tile-shape autotuner of the RHS stencil pass.
+"""Tile-shape autotuner of the stencil pass of two-pass plans.
 
     python -m sympygr_amd.autotune [--sizes 9 13 17 ...] [--top 6] [--dry-run]
 
@@ -7,7 +7,7 @@ stencil kernel admits (at most 512 points, halo and stage arrays within its
 LDS), ranks them by a cost model (points computed per interior point, halo
 loads, mixed-derivative stage cells and x-row length per tile point), times
 the best few and 8^3 on a uniform tiling of n^3 blocks (one
-RHS, FP64, upwind; SGR_TILE_SHAPE forces each shape), and keeps the fastest.
+RHS, mixed precision, upwind; SGR_TILE_SHAPE forces each shape), and keeps the fastest.
 It writes the table sgr_plan_create reads (default
 sympygr_amd/csrc/gen/tile_table.inc; rebuild the library afterwards) and a
 report with every timing (default profiles/tile_autotune.json).  Needs a GPU.
@@ -71,7 +71,7 @@ def time_shape(n, shape, steps=10):
     out = torch.zeros_like(u)
     os.environ["SGR_TILE_SHAPE"] = ",".join(str(x) for x in shape)
     try:
-        plan = sgr.Plan(bl, sgr.params(adv="upwind", precision="fp64", ko_sigma=0.1))
+        plan = sgr.Plan(bl, sgr.params(adv="upwind", precision="mixed", ko_sigma=0.1))
     finally:
         del os.environ["SGR_TILE_SHAPE"]
     for _ in range(2):
@@ -114,7 +114,7 @@ def main():
         return
     git = subprocess.run(["git", "rev-parse", "--short", "HEAD"], capture_output=True, text=True,
                          cwd=ROOT).stdout.strip() or None  # None outside a git checkout
-    report = {"git": git, "metric": "RHS Mpoints/s, FP64, upwind, uniform tiling of n^3 blocks (about 12 M points)",
+    report = {"git": git, "metric": "RHS Mpoints/s, mixed precision, upwind, uniform tiling of n^3 blocks (about 12 M points)",
               "sizes": {}}
     choice = {}
     for n in args.sizes:

@@ -1,8 +1,8 @@
 // BSSN (and CCZ4) RHS kernels for gfx950 (CDNA4).
 //
-// The FP64 BSSN right-hand side (standard gauge, Kreiss-Oliger) is one kernel,
-// k_rhs (one_pass.hip).  Mixed precision, CCZ4, the Rochester gauge and TVB
-// dissipation, and calls whose outputs overlap their inputs, are two passes
+// The FP64 right-hand side in the standard gauge is one kernel, k_rhs
+// (one_pass.h).  Mixed precision, the Rochester gauge and calls whose outputs
+// overlap their inputs are two passes
 // over interior tiles (8x8x8, or another shape for the block's size), with a
 // tile-major derivative workspace between them:
 //
