@@ -3,7 +3,7 @@
 // only after the divergence of Gamma-hat.  A 192^3 block with flagged faces:
 // 5.1 ms in two passes, 3.8 ms here.  Parking
 // Z^i and those two equations in LDS instead of registers removed the scratch
-// reloads of the field loops and still took 9% longer.
+// reloads of the field loops and still took 7% longer (4.02 -> 4.32 ms).
 #include "one_pass.h"
 
 namespace sgr {
