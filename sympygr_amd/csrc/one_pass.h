@@ -16,7 +16,7 @@
 //
 // so what a point carries from field to field is at most about 50 doubles and
 // nothing of it goes to memory.  512 blocks of 32^3 points took 11.9 ms in two
-// passes and take 7.4 ms here (10.7 and 6.3 ms without flagged faces).  What bounds it:
+// passes and take 7.3 ms here (10.7 and 6.3 ms without flagged faces).  What bounds it:
 // issue of FP64 and LDS instructions by two waves per SIMD that a barrier keeps
 // in step.
 #pragma once
@@ -670,6 +670,17 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
 
         bool own;  // is the point this tile's (tile_at)?
         int gp;    // its place in the block
+        // Stores of the points the tile owns.  MASKED: buffer stores from the tile's
+        // corner, the other points' offset out of range, which drops the lane.  Behind
+        // a branch the number of stores in flight is unknown to the compiler, and each
+        // wait for the next field's loads is one for the last field's stores too: 512 x
+        // 32^3 7.49 -> 7.28 ms, CCZ4 3% (general shapes 11%).  The general BSSN kernels
+        // spill scalar registers over it (33^3 blocks 1.36 -> 1.55 ms) and keep the
+        // branch.  (32 bits of offset: in and out arrays of a block with larger planes
+        // fit no device.)
+        constexpr bool MASKED = !GEN || (CCZ4 && !RK);
+        const uint64_t corner = tc.i0 + (uint64_t)n0 * (tc.j0 + (uint64_t)n1 * tc.k0);
+        uint32_t soff;
         {
             int lx, ly, lz;
             bool has;
@@ -677,7 +688,17 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
             const int pi = tc.i0 + lx, pj = tc.j0 + ly, pk = tc.k0 + lz;
             own = has && pi >= tc.oi && pj >= tc.oj && pk >= tc.ok;
             gp = pi + n0 * (pj + n1 * pk);
+            soff = own ? 8u * (uint32_t)(lx + n0 * (ly + n1 * lz)) : 0xFFFFFFF8u;
         }
+        auto store = [&](SGR_GLOBAL double *a, double k) __attribute__((always_inline)) {
+            if constexpr (!MASKED) {
+                if (own) a[gp] = k;
+                return;
+            }
+            typedef unsigned Words __attribute__((ext_vector_type(2)));
+            const auto r = __builtin_amdgcn_make_buffer_rsrc((void *)(uint64_t)(a + corner), 0, 0xFFFFFFF0u, 0x00027000);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Words, k), r, (int)soff, 0, 0);
+        };
         double bv[3], g[6], ig[6];
 #pragma unroll
         for (int d = 0; d < 3; d++) bv[d] = MONITOR ? 0.0 : pv[d];
@@ -841,18 +862,17 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
         };
         auto finish_value = [&](const FieldVals &v, double k) __attribute__((always_inline)) {
             SGR_EXACT
-            if (!own) return;
             if (!RK) {
-                v.out[gp] = k;
+                store(v.out, k);
                 return;
             }
             const double wk = rk.w * k;
             if (rk.stage == 3) {
-                v.next[gp] = v.acv + wk;
+                store(v.next, v.acv + wk);
                 return;
             }
-            v.out[gp] = (rk.stage == 0 ? v.u0v : v.acv) + wk;
-            v.next[gp] = v.u0v + rk.cn * k;
+            store(v.out, (rk.stage == 0 ? v.u0v : v.acv) + wk);
+            store(v.next, v.u0v + rk.cn * k);
         };
         auto finish = [&](const FieldVals &v, double alg, double lin) __attribute__((always_inline)) {
             SGR_EXACT
