@@ -155,8 +155,10 @@ int tile_shape(const sgr_block &b, bool one_pass, bool few, int td[3])
             }
         }
     }
-    // no tile reaches beyond its block (k_rhs reads whole halo tiles)
-    for (int k = 0; k < 3; k++) td[k] = std::min(td[k], (int)b.sz[k] - 6);
+    // no tile of the one-pass kernels reaches beyond its block: they read whole
+    // halo tiles (the two passes check; 7^3 blocks as 8^3 tiles take 0.87 of the
+    // time of the general kernel in mixed precision)
+    for (int k = 0; k < 3 && one_pass; k++) td[k] = std::min(td[k], (int)b.sz[k] - 6);
     return SGR_OK;
 }
 
@@ -464,6 +466,7 @@ struct sgr_plan {
     uint32_t cchunk_tiles = 0;   // tiles per constraint launch
     uint64_t ws_bytes = 0;
     uint64_t interior = 0;
+    bool inside = true;  // no RHS tile reaches beyond its block
     std::array<TileList, 2> all{};  // one-pass constraints: the plan's 8^3 tiles, and its others
     std::vector<std::array<TileList, 2>> lists;  // one-pass RHS: each chunk's 8^3 tiles, and its others
     uint64_t span = 0;           // nodes of a field array the blocks reach
@@ -570,6 +573,7 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
             return rc;
         }
         p->hblocks.push_back(block_desc(blocks[b], &shape[3 * b], 0, 0));
+        for (int k = 0; k < 3; k++) p->inside = p->inside && shape[3 * b + k] <= (int)blocks[b].sz[k] - 6;
         p->interior += (uint64_t)(blocks[b].sz[0] - 6) * (blocks[b].sz[1] - 6) * (blocks[b].sz[2] - 6);
         p->span = std::max<uint64_t>(p->span, blocks[b].offset + (uint64_t)blocks[b].sz[0] * blocks[b].sz[1] *
                                                                      blocks[b].sz[2]);
@@ -940,7 +944,8 @@ static int constraints_impl(sgr_plan *plan, const double *const in[SGR_NUM_VARS]
     }
     // one kernel, unless an output shares memory with an input: its points are
     // written while their neighbours' stencils may still read them
-    bool fused = true;
+    // (nor with a tile that reaches beyond its block: two-pass plans, blocks of 7)
+    bool fused = plan->inside;
     for (int f = 0; f < NF; f++)
         for (int c = 0; c < (psi4 ? 6 : 4); c++) fused = fused && !arrays_meet(in[f], out[c], plan->span);
     a.blocks = plan->d_blocks;
