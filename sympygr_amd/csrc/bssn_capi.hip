@@ -867,7 +867,7 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
     for (int q = 0; q < 4; q++) a.ev[q] = ev ? ev[q] : nullptr;
     a.rk.stage = -1;
     if (rk) a.rk = *rk;
-    a.fused = one_pass_call(plan->params, a.in, a.out, a.rk, plan->span);
+    a.fused = !plan->lists.empty() && one_pass_call(plan->params, a.in, a.out, a.rk, plan->span);
     if (plan->params.dissipation != SGR_DISS_KO) {
         // TVB replaces the Kreiss-Oliger term: the stencil pass leaves it out
         // of the tails and k_tvb adds sigma (D_x + D_y + D_z) to them
@@ -886,7 +886,7 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
     } else if (a.fused && plan->lists.size() > 1) {
         e = one_pass_chunks(plan, a, stream, ev);
     } else if (e == hipSuccess && plan->ntiles <= plan->chunk_tiles) {
-        if (a.fused && plan->ntiles)
+        if (a.fused)
             for (int k = 0; k < 2; k++) a.list[k] = plan->lists[0][k];
         e = launch_rhs(a, stream);
     } else if (e == hipSuccess && plan->pipe) {
@@ -1165,10 +1165,10 @@ int sgr_check_finite(sgr_plan *plan, const double *const in[SGR_NUM_VARS], hipSt
 // (an OpenMP loop over blocks), so every calling thread keeps its own staging
 // context: a one-block plan, a stream of its own and its device and pinned
 // host buffers.  The plan is rebuilt only when the device, the block size or
-// the kernel-selecting parameters (advection, precision) change; the block's
-// offset, coordinates and bflag are uploaded with each call.  Contexts of
-// different threads run concurrently on the GPU; each is held until its
-// thread ends.
+// a parameter that its tiles, lists and arrays depend on changes (stage_plan);
+// the block's offset, coordinates and bflag are uploaded with each call.
+// Contexts of different threads run concurrently on the GPU; each is held
+// until its thread ends.
 namespace {
 struct BlockStage {
     sgr_plan *plan = nullptr;
@@ -1220,6 +1220,7 @@ int stage_plan(const sgr_block &b, const sgr_params *params, int device)
     const bool same = S.plan && S.sz[0] == b.sz[0] && S.sz[1] == b.sz[1] && S.sz[2] == b.sz[2] &&
                       S.adv == params->adv_mode && S.prec == params->precision &&
                       S.plan->params.formulation == params->formulation &&
+                      one_pass(S.plan->params) == one_pass(*params) &&    // decides tile shapes and tile lists
                       S.plan->params.dissipation == params->dissipation;  // TVB plans hold the speed arrays
     if (!same) {
         if (S.plan) {
