@@ -1166,7 +1166,7 @@ int sgr_check_finite(sgr_plan *plan, const double *const in[SGR_NUM_VARS], hipSt
 // context: a one-block plan, a stream of its own and its device and pinned
 // host buffers.  The plan is rebuilt only when the device, the block size or
 // a parameter that its tiles, lists and arrays depend on changes (stage_plan);
-// the block's offset, coordinates and bflag are uploaded with each call.
+// the block's coordinates and bflag are uploaded with each call.
 // Contexts of different threads run concurrently on the GPU; each is held
 // until its thread ends.
 namespace {
@@ -1202,8 +1202,8 @@ struct BlockStage {
 };
 thread_local BlockStage g_stage;
 
-// The context's plan set up for block b (sz, offset, geometry) and params
-// on `device`, and its stream; the device is current.
+// The context's plan set up for block b (at offset 0) and params on `device`,
+// and its stream; the device is current.
 int stage_plan(const sgr_block &b, const sgr_params *params, int device)
 {
     BlockStage &S = g_stage;
@@ -1235,18 +1235,16 @@ int stage_plan(const sgr_block &b, const sgr_params *params, int device)
         S.prec = params->precision;
         return SGR_OK;
     }
-    // same size: new offset, coordinates, bflag and physics parameters; the
-    // descriptor goes up on the context's stream, ahead of the kernels
+    // same size: new coordinates, bflag and physics parameters; the descriptor
+    // goes up on the context's stream, ahead of the kernels
     HIP_TRY(hipStreamSynchronize(S.stream), "hipStreamSynchronize");  // the pinned copy is free again
     BlockDesc &d = S.plan->hblocks[0];
-    d.offset = b.offset;
     d.bflag = b.bflag;
     for (int k = 0; k < 3; k++) {
         d.pmin[k] = b.pmin[k];
         d.ax[k] = axis_const(b.pmin[k], b.pmax[k], b.sz[k]);
     }
     S.plan->params = *params;
-    S.plan->span = b.offset + (uint64_t)b.sz[0] * b.sz[1] * b.sz[2];
     S.plan->use_queue = stencil_queue(face_tiles(d), S.plan->ntiles);
     *S.h_desc = d;
     HIP_TRY(hipMemcpyAsync(S.plan->d_blocks, S.h_desc, sizeof(BlockDesc), hipMemcpyHostToDevice, S.stream),
@@ -1298,14 +1296,24 @@ int sgr_rhs_block(double *const out[SGR_NUM_VARS], const double *const in[SGR_NU
                   const sgr_params *params, int device)
 {
     if (!out || !in) return fail(SGR_E_INVALID, "null argument");
+    // The kept plan's block lies at offset 0 and the arrays start at the block:
+    // what the plan sizes by the nodes its blocks reach (the characteristic
+    // speeds of TVB dissipation) then fits every block of the size.
     sgr_block b;
-    int rc = block_checks(pmin, pmax, sz, bflag, params, offset, b);
+    int rc = block_checks(pmin, pmax, sz, bflag, params, 0, b);
     if (rc) return rc;
+    const double *i[NFMAX];
+    double *o[NFMAX];
+    for (int f = 0; f < (params->formulation == SGR_FORM_CCZ4 ? NF_CCZ4 : NF); f++) {
+        if (!in[f] || !out[f]) return fail(SGR_E_INVALID, "null field pointer");
+        i[f] = in[f] + offset;
+        o[f] = out[f] + offset;
+    }
     int cur = 0;
     hipGetDevice(&cur);
     HIP_TRY(hipSetDevice(device), "hipSetDevice");
     rc = stage_plan(b, params, device);
-    if (rc == SGR_OK) rc = sgr_rhs(g_stage.plan, out, in, g_stage.stream);
+    if (rc == SGR_OK) rc = sgr_rhs(g_stage.plan, o, i, g_stage.stream);
     if (rc == SGR_OK) {
         hipError_t e = hipStreamSynchronize(g_stage.stream);
         if (e != hipSuccess) rc = hip_fail(e, "hipStreamSynchronize");

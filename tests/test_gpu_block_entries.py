@@ -64,3 +64,26 @@ def test_gauge_changes_between_blocks_of_one_size(n, gib, host, monkeypatch):
             ref = po.rhs_block(u, sz, pmin, pmax, 63, po.make_params(upwind=True, **kw))
             assert normwise(interior(got, sz), interior(ref, sz)).max() <= 1e-12, (k, gauge)
     _in_new_thread(calls)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("diss", ["tvb3", "tvb5"])
+def test_tvb_blocks_at_growing_offsets(diss, precision):
+    """Equal-sized blocks one after another out of one set of arrays, as a
+    block loop calls them: each reads the characteristic speeds of its own
+    nodes, so all equal the plan over the whole set bit for bit."""
+    import torch
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    bl = data.uniform_tiling(nb=2, n=16, lo=-1.0, hi=1.0, stagger=0.5, faces=True)
+    u = data.fill_blocks(bl, backend="torch", device="cuda", kind="perturbed", seed=8, amp=1e-2, lo=-1.0, L=2.0)
+    prm = sgr.params(adv="upwind", ko_sigma=0.1, dissipation=diss, precision=precision)
+    out, ref = torch.full_like(u, 5.0), torch.full_like(u, 5.0)
+    sgr.Plan(bl, prm).rhs(ref, u)
+    torch.cuda.synchronize()
+
+    def calls():
+        for b in range(len(bl)):
+            sgr.rhs_block(out, u, bl.offsets[b], bl.pmin[b], bl.pmax[b], bl.sz[b], bl.bflag[b], prm)
+    _in_new_thread(calls)
+    assert torch.equal(out, ref)
