@@ -352,10 +352,11 @@ def bssnrhs(out, u, offset, pmin, pmax, sz, bflag, prm: SgrParams, device=0):
 
 def rhs_block(out, u, offset, pmin, pmax, sz, bflag, prm: SgrParams, device=0):
     """sgr_rhs_block: the reference bssnrhs (bssn/include/rhs.h:33-36) on
-    device tensors u, out of shape (24, N), synchronous; reads the padded
-    block at `offset`, writes its interior RHS into `out`."""
+    device tensors u, out of shape (24, N) (CCZ4: (25, N)), synchronous; reads
+    the padded block at `offset`, writes its interior RHS into `out`."""
+    nf = NUM_VARS_CCZ4 if prm.formulation == FORM["ccz4"] else NUM_VARS
     need = offset + sz[0] * sz[1] * sz[2]
-    check(lib().sgr_rhs_block(_field_ptrs(out, need, device), _field_ptrs(u, need, device), offset,
+    check(lib().sgr_rhs_block(_rows(out, nf, need, device), _rows(u, nf, need, device), offset,
                               (ctypes.c_double * 3)(*pmin),
                               (ctypes.c_double * 3)(*pmax), (ctypes.c_uint32 * 3)(*sz), bflag,
                               ctypes.byref(prm), device))

@@ -87,3 +87,22 @@ def test_tvb_blocks_at_growing_offsets(diss, precision):
             sgr.rhs_block(out, u, bl.offsets[b], bl.pmin[b], bl.pmax[b], bl.sz[b], bl.bflag[b], prm)
     _in_new_thread(calls)
     assert torch.equal(out, ref)
+
+
+def test_ccz4_block_takes_25_fields():
+    """A CCZ4 block has a 25th array: 24 are refused before the library would
+    read a pointer that is not there."""
+    import torch
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    bl = data.BlockList()
+    bl.add((22, 22, 22), (-1.05,) * 3, (1.05,) * 3, 63)
+    u = data.fill_blocks(bl, backend="torch", device="cuda", kind="ccz4", seed=4, amp=1e-2, lo=-1.05, L=2.1)
+    prm = sgr.params(adv="upwind", formulation="ccz4")
+    ref, got = torch.full_like(u, 5.0), torch.full_like(u, 5.0)
+    sgr.Plan(bl, prm).rhs(ref, u)
+    torch.cuda.synchronize()
+    sgr.rhs_block(got, u, 0, bl.pmin[0], bl.pmax[0], bl.sz[0], 63, prm)
+    assert torch.equal(got, ref)
+    with pytest.raises(ValueError, match="25"):
+        sgr.rhs_block(got[:24], u[:24], 0, bl.pmin[0], bl.pmax[0], bl.sz[0], 63, prm)
