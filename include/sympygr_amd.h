@@ -142,7 +142,10 @@ int sgr_plan_get_info(const sgr_plan *plan, sgr_plan_info *info);
  * captured into a HIP graph.  A pipelined plan (sgr_plan_info) also runs
  * work on its own second stream, forked from and joined back into `stream`
  * through events, so the call is ordered on `stream` as one launch would
- * be.  Calls on one plan share its workspace (and second stream) and must
+ * be.  out[f] may be in[f] itself (in place; SGR_E_INVALID if the plan runs
+ * in several workspace chunks and its workspace does not hold the largest
+ * block); any other output must not share memory with a block's input.
+ * Calls on one plan share its workspace (and second stream) and must
  * not overlap: issue them on one stream or serialise them.  Replaces the
  * reference's multi-block entry bssnRHS (bssn/include/rhs.h:31) and its GPU
  * plug-in cuda::computeRHS (bssn/cuda_gr/include/rhs_cuda.cuh:39). */

@@ -263,21 +263,50 @@ bool arrays_meet(const double *a, const double *b, uint64_t span)
     return (x < y ? y - x : x - y) < span * sizeof(double);
 }
 
-// Whether one RHS call does: such parameters, and no output array shares
-// memory with an input array (k_rhs writes a point while its neighbours'
-// stencils may still read it; the two passes do not).  span: nodes of a field
-// array that the blocks reach.
-bool one_pass_call(const sgr_params &p, const FieldPtrs &in, const OutPtrs &out, const RkArgs &rk, uint64_t span)
+// How the output arrays of a call lie to its input arrays.
+enum class Lie {
+    APART,  // no output shares memory with an input: k_rhs (which writes a point while its
+            // neighbours' stencils may still read it) can run
+    MEET,   // the ranges of two arrays do, but no output is an input (arrays whose blocks
+            // lie between each other's)
+    OVER,   // an output array is an input array
+};
+
+// span: nodes of a field array that the blocks reach.
+Lie outputs_lie(const FieldPtrs &in, const OutPtrs &out, const RkArgs &rk, int nf, uint64_t span)
 {
-    if (!one_pass(p)) return false;
-    auto meets = [&](const double *a, const double *b) { return arrays_meet(a, b, span); };
-    const int nf = p.formulation == SGR_FORM_CCZ4 ? NF_CCZ4 : NF;
+    Lie lie = Lie::APART;
+    auto look = [&](const double *a, const double *b) {
+        if (a == b) lie = Lie::OVER;
+        else if (lie == Lie::APART && arrays_meet(a, b, span)) lie = Lie::MEET;
+    };
     for (int f = 0; f < nf; f++)
         for (int g = 0; g < nf; g++) {
-            if (meets(in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g])) return false;
-            if (rk.stage >= 0 && rk.stage < 3 && meets(in.p[f], rk.acc.p[g])) return false;
+            look(in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g]);
+            if (rk.stage >= 0 && rk.stage < 3) look(in.p[f], rk.acc.p[g]);
         }
-    return true;
+    return lie;
+}
+
+// The last tile (exclusive) of each launch when launches hold whole blocks only:
+// as many as `cap` tiles of workspace take; none if a block has more.  Outputs
+// over inputs run like that: a block's stencils read its own nodes, so what an
+// earlier launch has overwritten is not read any more.
+// nt: a block's tiles per axis (BlockDesc::ntile or ntile8).
+std::vector<uint32_t> block_cuts(const std::vector<BlockDesc> &hb, const std::vector<uint32_t> &tile_block,
+                                 int32_t (BlockDesc::*nt)[3], uint64_t cap)
+{
+    std::vector<uint32_t> cuts;
+    uint64_t first = 0;  // tile of the current launch
+    for (uint64_t i = 0; i < tile_block.size();) {
+        const int32_t *t = hb[tile_block[i]].*nt;
+        const uint64_t n = (uint64_t)t[0] * t[1] * t[2];
+        if (n > cap) return {};
+        if (i + n - first > cap) cuts.push_back((uint32_t)i), first = i;
+        i += n;
+    }
+    if (!tile_block.empty()) cuts.push_back((uint32_t)tile_block.size());
+    return cuts;
 }
 
 // Which RHS tiles come within three points of a flagged face (where k_rhs takes
@@ -465,6 +494,7 @@ struct sgr_plan {
     uint32_t chunk_tiles = 0;    // tiles per RHS launch (workspace capacity)
     uint32_t cchunk_tiles = 0;   // tiles per constraint launch
     uint64_t ws_bytes = 0;
+    std::vector<uint32_t> cuts;  // RHS launches of whole blocks (block_cuts)
     uint64_t interior = 0;
     bool inside = true;  // no RHS tile reaches beyond its block
     std::array<TileList, 2> all{};  // one-pass constraints: the plan's 8^3 tiles, and its others
@@ -652,6 +682,7 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
         tile_block8.insert(tile_block8.end(), nt, b);
     }
     p->ntiles = (uint32_t)tile_block.size();
+    p->cuts = block_cuts(p->hblocks, tile_block, &BlockDesc::ntile, p->ws_bytes / rhs_tile);
     std::vector<uint32_t> order;
     const std::vector<uint8_t> slow = closure_tiles(p->hblocks, tile_block);
     if (p->ntiles) {
@@ -867,7 +898,12 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
     for (int q = 0; q < 4; q++) a.ev[q] = ev ? ev[q] : nullptr;
     a.rk.stage = -1;
     if (rk) a.rk = *rk;
-    a.fused = !plan->lists.empty() && one_pass_call(plan->params, a.in, a.out, a.rk, plan->span);
+    const Lie lie = outputs_lie(a.in, a.out, a.rk, plan->nf, plan->span);
+    a.fused = one_pass(plan->params) && !plan->lists.empty() && lie == Lie::APART;
+    const bool whole = lie == Lie::OVER && plan->ntiles > plan->chunk_tiles;  // launches of whole blocks
+    if (whole && plan->cuts.empty())
+        return fail(SGR_E_INVALID, "an output array is an input array, and the plan's workspace does not hold a whole "
+                                   "block: pass separate output arrays (or raise SGR_WS_GIB)");
     if (plan->params.dissipation != SGR_DISS_KO) {
         // TVB replaces the Kreiss-Oliger term: the stencil pass leaves it out
         // of the tails and k_tvb adds sigma (D_x + D_y + D_z) to them
@@ -889,17 +925,18 @@ static int rhs_impl(sgr_plan *plan, double *const out[SGR_NUM_VARS], const doubl
         if (a.fused)
             for (int k = 0; k < 2; k++) a.list[k] = plan->lists[0][k];
         e = launch_rhs(a, stream);
-    } else if (e == hipSuccess && plan->pipe) {
+    } else if (e == hipSuccess && plan->pipe && !whole) {
         e = pipelined(plan, a, stream, ev);
     } else if (e == hipSuccess) {
         // several workspace chunks: events[0..1] bracket the whole call,
         // events[2..3] are recorded at its end
         if (ev) e = hipEventRecord(ev[0], stream);
         for (int q = 0; q < 4; q++) a.ev[q] = nullptr;
-        for (uint32_t t0 = 0; e == hipSuccess && t0 < plan->ntiles; t0 += plan->chunk_tiles) {
+        for (uint32_t t0 = 0, c = 0; e == hipSuccess && t0 < plan->ntiles; t0 += a.ntiles, c++) {
             a.tile0 = t0;
-            a.ntiles = plan->ntiles - t0 < plan->chunk_tiles ? plan->ntiles - t0 : plan->chunk_tiles;
+            a.ntiles = whole ? plan->cuts[c] - t0 : std::min(plan->ntiles - t0, plan->chunk_tiles);
             a.nfast = plan->nfast <= t0 ? 0 : std::min(plan->nfast - t0, a.ntiles);
+            if (whole) a.wsT = (double *)((char *)plan->d_ws + (uint64_t)a.ntiles * TILE_PTS * rs_nslot(plan->nf) * plan->wsz);
             e = launch_rhs(a, stream);
         }
         if (e == hipSuccess && ev) e = hipEventRecord(ev[1], stream);
@@ -1455,7 +1492,8 @@ int sgr_rhs_block_noalloc(double *const out[SGR_NUM_VARS], const double *const i
         a.out.p[f] = out[f];
     }
     a.rk.stage = -1;
-    a.fused = one_pass_call(*params, a.in, a.out, a.rk, offset + (uint64_t)sz[0] * sz[1] * sz[2]);
+    a.fused = one_pass(*params) &&
+              outputs_lie(a.in, a.out, a.rk, nf, offset + (uint64_t)sz[0] * sz[1] * sz[2]) == Lie::APART;
     if (a.fused) {  // (needs the map of its tiles only; the refusal above stays that of the two passes)
         rc = tile_shape(b, true, cube_tiles(b) <= FEW_TILES, td);
         if (rc) return rc;

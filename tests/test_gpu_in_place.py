@@ -1,0 +1,100 @@
+"""Outputs over inputs: the two-pass kernels, in launches of whole blocks, since
+a block's stencils must read its nodes before any launch overwrites them."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(bl, prm, monkeypatch, pipe=None, gib=None):
+    import sympygr_amd as sgr
+    for k, v in (("SGR_PIPE_CHUNKS", pipe), ("SGR_WS_GIB", gib)):
+        if v is None:
+            monkeypatch.delenv(k, raising=False)
+        else:
+            monkeypatch.setenv(k, v)
+    plan = sgr.Plan(bl, prm)
+    for k in ("SGR_PIPE_CHUNKS", "SGR_WS_GIB"):
+        monkeypatch.delenv(k, raising=False)
+    return plan
+
+
+def _tiling(kind, sizes=(16, 17)):
+    """Blocks of two sizes in turn (8^3 tiles and, in two-pass plans, tiles of
+    another shape), all faces of half of them flagged."""
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    bl = data.BlockList()
+    for b in range(8):
+        n = sizes[b % 2] + 6
+        lo = (-1.0 + 0.1 * b, -0.5, -0.7)
+        bl.add((n, n, n), lo, tuple(v + 0.04 * (n - 1) for v in lo), 63 if b & 2 else 0)
+    kw = dict(adv="upwind", ko_sigma=0.1)
+    if kind == "mixed":
+        kw["precision"] = "mixed"
+    elif kind == "ccz4":
+        kw["formulation"] = "ccz4"
+    elif kind == "tvb5":
+        kw["dissipation"] = "tvb5"
+    u = data.fill_blocks(bl, backend="torch", device="cuda", kind="ccz4" if kind == "ccz4" else "perturbed", seed=5,
+                         amp=1e-2, lo=-1.0, L=2.0)
+    return bl, u, sgr.params(**kw)
+
+
+@pytest.mark.parametrize("kind", ["fp64", "mixed", "ccz4", "tvb5"])
+def test_rhs_in_place_in_several_launches(kind, monkeypatch):
+    """In place over several workspace chunks, consecutive and pipelined: the
+    bits of in place in one launch, and to rounding the right-hand side of
+    separate arrays (1e-12 of each field's maximum; mixed precision runs the
+    same kernels there: equal).  A workspace that does not hold the largest
+    block is refused."""
+    import torch
+    import sympygr_amd as sgr
+    bl, u, prm = _tiling(kind)
+    one = _plan(bl, prm, monkeypatch)
+    assert one.info().chunks == 1
+    ref, sep = u.clone(), u.clone()
+    one.rhs(ref, ref)
+    one.rhs(sep, u)
+    torch.cuda.synchronize()
+    if kind == "mixed":
+        assert torch.equal(ref, sep)
+    for f in range(u.shape[0]):  # (ghost nodes hold the inputs in both)
+        inner = sep[f] != u[f]
+        assert (ref[f] - sep[f]).abs().max() <= 1e-12 * sep[f][inner].abs().max(), f
+    nf = u.shape[0]
+    tile = 512 * ((one.info().derivative_slots - nf) * (4 if kind == "mixed" else 8) + nf * 8)  # workspace of a tile
+    largest = one.info().tiles // 4 - 8  # four blocks of 16^3 (8 tiles each), four of 17^3
+    ran = 0
+    for pipe, gib in (("0", "0.01"), (None, "0.01"), ("5", None)):
+        plan = _plan(bl, prm, monkeypatch, pipe, gib)
+        info = plan.info()
+        fits = info.workspace_bytes >= largest * tile
+        print(f"{kind}: chunks={info.chunks} pipelined={info.pipelined} fits={fits}", flush=True)
+        assert info.chunks > 1
+        got = u.clone()
+        if not fits:
+            with pytest.raises(sgr.SgrError, match="separate output arrays"):
+                plan.rhs(got, got)
+            continue
+        ran += 1
+        plan.rhs(got, got)
+        torch.cuda.synchronize()
+        assert torch.equal(got, ref), (pipe, gib)
+    assert ran
+
+
+def test_rhs_in_place_refused_if_a_block_does_not_fit(monkeypatch):
+    """A workspace of fewer tiles than a block has: refused, nothing written;
+    the same plan takes separate arrays."""
+    import torch
+    import sympygr_amd as sgr
+    bl, u, prm = _tiling("fp64", sizes=(24, 13))
+    plan = _plan(bl, prm, monkeypatch, None, "0.004")
+    got = u.clone()
+    with pytest.raises(sgr.SgrError, match="separate output arrays"):
+        plan.rhs(got, got)
+    out, ref = torch.full_like(u, 5.0), torch.full_like(u, 5.0)
+    plan.rhs(out, u)
+    _plan(bl, prm, monkeypatch).rhs(ref, u)
+    torch.cuda.synchronize()
+    assert torch.equal(got, u) and torch.equal(out, ref)
