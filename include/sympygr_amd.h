@@ -169,7 +169,11 @@ int sgr_rhs_events(sgr_plan *plan, double *const out[SGR_NUM_VARS], const double
  * derivatives are staged in the plan's workspace type: FP64 for an FP64
  * plan; FP32 for a mixed-precision plan, whose constraints therefore carry
  * FP32 rounding of the derivatives (about 1e-7 relative) -- use an FP64 plan
- * for FP64 constraints.  Uses the plan's workspace: do not overlap with
+ * for FP64 constraints.  An output may be one of the input arrays (if it is
+ * one that the constraints read, all but the lapse, the shift and B:
+ * SGR_E_INVALID unless the plan's workspace holds the largest block's
+ * derivatives); any other output must not share memory with a block's input.
+ * Uses the plan's workspace: do not overlap with
  * sgr_rhs on the same plan.  The reference's generated counterpart
  * (bssn/CodeGen/physcon.cpp) does not compile. */
 int sgr_constraints(sgr_plan *plan, const double *const in[SGR_NUM_VARS], double *const out[4], hipStream_t stream);

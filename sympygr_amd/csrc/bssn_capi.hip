@@ -272,18 +272,21 @@ enum class Lie {
     OVER,   // an output array is an input array
 };
 
-// span: nodes of a field array that the blocks reach.
+// `lie` with one more input and output array; span: nodes of a field array that
+// the blocks reach.
+void look(Lie &lie, const double *in, const double *out, uint64_t span)
+{
+    if (in == out) lie = Lie::OVER;
+    else if (lie == Lie::APART && arrays_meet(in, out, span)) lie = Lie::MEET;
+}
+
 Lie outputs_lie(const FieldPtrs &in, const OutPtrs &out, const RkArgs &rk, int nf, uint64_t span)
 {
     Lie lie = Lie::APART;
-    auto look = [&](const double *a, const double *b) {
-        if (a == b) lie = Lie::OVER;
-        else if (lie == Lie::APART && arrays_meet(a, b, span)) lie = Lie::MEET;
-    };
     for (int f = 0; f < nf; f++)
         for (int g = 0; g < nf; g++) {
-            look(in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g]);
-            if (rk.stage >= 0 && rk.stage < 3) look(in.p[f], rk.acc.p[g]);
+            look(lie, in.p[f], rk.stage < 0 ? out.p[g] : rk.next.p[g], span);
+            if (rk.stage >= 0 && rk.stage < 3) look(lie, in.p[f], rk.acc.p[g], span);
         }
     return lie;
 }
@@ -494,7 +497,7 @@ struct sgr_plan {
     uint32_t chunk_tiles = 0;    // tiles per RHS launch (workspace capacity)
     uint32_t cchunk_tiles = 0;   // tiles per constraint launch
     uint64_t ws_bytes = 0;
-    std::vector<uint32_t> cuts;  // RHS launches of whole blocks (block_cuts)
+    std::vector<uint32_t> cuts, cuts8;  // RHS and constraint launches of whole blocks (block_cuts)
     uint64_t interior = 0;
     bool inside = true;  // no RHS tile reaches beyond its block
     std::array<TileList, 2> all{};  // one-pass constraints: the plan's 8^3 tiles, and its others
@@ -705,6 +708,7 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
     }
     tile_block.insert(tile_block.end(), order.begin(), order.end());
     p->ntiles8 = (uint32_t)tile_block8.size();
+    p->cuts8 = block_cuts(p->hblocks, tile_block8, &BlockDesc::ntile8, p->ws_bytes / con_tile);
     // optional cap on the plan's device memory (SGR_DEVICE_MEM_LIMIT_GIB):
     // a plan that would need more is refused before anything is allocated
     {
@@ -979,12 +983,17 @@ static int constraints_impl(sgr_plan *plan, const double *const in[SGR_NUM_VARS]
         if (!out[c]) return fail(SGR_E_INVALID, "null constraint pointer");
         co.p[c] = out[c];
     }
-    // one kernel, unless an output shares memory with an input: its points are
-    // written while their neighbours' stencils may still read them
-    // (nor with a tile that reaches beyond its block: two-pass plans, blocks of 7)
-    bool fused = plan->inside;
-    for (int f = 0; f < NF; f++)
-        for (int c = 0; c < (psi4 ? 6 : 4); c++) fused = fused && !arrays_meet(in[f], out[c], plan->span);
+    // one kernel, unless an output shares memory with an input that it reads (the
+    // lapse, the shift and B are not) or a tile reaches beyond its block (two-pass
+    // plans, blocks of 7); over an input, the two passes in launches of whole blocks
+    Lie lie = Lie::APART;
+    for (int f = 1; f < NF; f++)
+        for (int c = 0; c < (psi4 ? 6 : 4) && (f < 6 || f > 11); c++) look(lie, in[f], out[c], plan->span);
+    const bool fused = plan->inside && lie == Lie::APART;
+    const bool whole = lie == Lie::OVER && plan->ntiles8 > plan->cchunk_tiles;
+    if (whole && plan->cuts8.empty())
+        return fail(SGR_E_INVALID, "an output array is an input array that the constraints read, and the plan's workspace "
+                                   "does not hold a whole block: pass separate output arrays");
     a.blocks = plan->d_blocks;
     a.tile_block = fused ? plan->d_tile_block : plan->d_tile_block8;
     a.grid_cap = plan->grid_cap;
@@ -1000,9 +1009,9 @@ static int constraints_impl(sgr_plan *plan, const double *const in[SGR_NUM_VARS]
     if (cur != plan->device) HIP_TRY(hipSetDevice(plan->device), "hipSetDevice");
     hipError_t e = hipSuccess;
     if (fused) e = launch_monitor(a, co, psi4, stream);
-    for (uint32_t t0 = 0; !fused && e == hipSuccess && t0 < plan->ntiles8; t0 += plan->cchunk_tiles) {
+    for (uint32_t t0 = 0, c = 0; !fused && e == hipSuccess && t0 < plan->ntiles8; t0 += a.ntiles, c++) {
         a.tile0 = t0;
-        a.ntiles = plan->ntiles8 - t0 < plan->cchunk_tiles ? plan->ntiles8 - t0 : plan->cchunk_tiles;
+        a.ntiles = whole ? plan->cuts8[c] - t0 : std::min(plan->ntiles8 - t0, plan->cchunk_tiles);
         e = launch_constraints(a, co, psi4, stream);
     }
     if (cur != plan->device) hipSetDevice(cur);

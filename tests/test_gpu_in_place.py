@@ -98,3 +98,60 @@ def test_rhs_in_place_refused_if_a_block_does_not_fit(monkeypatch):
     _plan(bl, prm, monkeypatch).rhs(ref, u)
     torch.cuda.synchronize()
     assert torch.equal(got, u) and torch.equal(out, ref)
+
+
+def _rows_rel(bl, a, b):
+    """max |a - b| over the interior nodes, over each row's max |b|."""
+    import torch
+    d, m = [], []
+    for i in range(len(bl)):
+        s = bl.sz[i]
+        o = slice(bl.offsets[i], bl.offsets[i] + s[0] * s[1] * s[2])
+        x, y = (v[:, o].reshape(-1, s[2], s[1], s[0])[:, 3:-3, 3:-3, 3:-3] for v in (a, b))
+        d.append((x - y).abs().amax(dim=(1, 2, 3)))
+        m.append(y.abs().amax(dim=(1, 2, 3)))
+    return (torch.stack(d).amax(0) / torch.stack(m).amax(0)).max().item()
+
+
+@pytest.mark.parametrize("kind", ["fp64", "mixed"])
+@pytest.mark.parametrize("psi4,row", [(False, 12), (False, 1), (True, 18), (True, 12), (True, 6)])
+def test_constraints_over_inputs(kind, psi4, row, monkeypatch):
+    """Over rows that the constraints read (gt, At, chi to Gt) in several
+    launches, and over rows that they do not (shift and B): the values of
+    separate output arrays, to the bounds that both keep against the oracle,
+    1e-11 of a row's maximum and 1e-5 in mixed precision."""
+    import torch
+    bl, u, prm = _tiling(kind)
+    plan = _plan(bl, prm, monkeypatch)
+    n = 6 if psi4 else 4
+    sep = torch.full((n, u.shape[1]), 5.0, dtype=torch.float64, device="cuda")
+    over = u.clone()
+    call = plan.constraints_psi4 if psi4 else plan.constraints
+    call(u, sep)
+    call(over, over[row:row + n])
+    torch.cuda.synchronize()
+    assert _rows_rel(bl, over[row:row + n], sep) <= (1e-5 if kind == "mixed" else 1e-11)
+    rest = [f for f in range(24) if not row <= f < row + n]
+    assert torch.equal(over[rest], u[rest])
+
+
+def test_constraints_over_inputs_refused_if_a_block_does_not_fit(monkeypatch):
+    """One block of 27 tiles: its workspace holds the right-hand side's
+    derivatives of them, not the constraints'."""
+    import torch
+    import sympygr_amd as sgr
+    from sympygr_amd import data
+    bl = data.BlockList()
+    bl.add((30, 30, 30), (-0.7, -0.5, -0.6), (0.46, 0.66, 0.56), 0)
+    u = data.fill_blocks(bl, backend="torch", device="cuda", kind="perturbed", seed=5, amp=1e-2, lo=-1.0, L=2.0)
+    plan = sgr.Plan(bl, sgr.params(adv="upwind"))
+    over = u.clone()
+    with pytest.raises(sgr.SgrError, match="separate output arrays"):
+        plan.constraints(over, over[12:16])
+    torch.cuda.synchronize()
+    assert torch.equal(over, u)
+    sep = torch.zeros((4, bl.total), dtype=torch.float64, device="cuda")
+    plan.constraints(u, sep)
+    plan.constraints(over, over[8:12])
+    torch.cuda.synchronize()
+    assert _rows_rel(bl, over[8:12], sep) <= 1e-11
