@@ -882,14 +882,18 @@ __global__ __launch_bounds__(256) void k_constraints(FieldPtrs in, OutPtrs cout,
 #define BSSN_D2(F_, S_) ((R)ws_get(&wsb[slot_d2(F_, S_) * SS]))
 #define BSSN_LAP(F_) ((R)ws_get(&wsb[slot_lap(F_) * SS]))
 #define BSSN_GDB(J_) ((R)ws_get(&wsb[slot_gdb(J_) * SS]))
-#define BSSN_OUT(C_, V_) cout.p[C_][pp] = (V_)
+#define BSSN_OUT(C_, V_) cv[C_] = (V_)
 #define BSSN_BARRIER()
+    // (stored when every input is read: an output may be an input array)
+    R cv[PSI4 ? 6 : 4];
     if constexpr (PSI4) {
         const R px = B.pmin[0] + i * B.ax[0].h, py = B.pmin[1] + j * B.ax[1].h, pz = B.pmin[2] + k * B.ax[2].h;
 #include "gen/bssn_constraints_psi4.inc"
     } else {
 #include "gen/bssn_constraints.inc"
     }
+#pragma unroll
+    for (int c = 0; c < (PSI4 ? 6 : 4); c++) cout.p[c][pp] = cv[c];
 #undef BSSN_U
 #undef BSSN_D1
 #undef BSSN_D2

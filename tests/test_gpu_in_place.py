@@ -114,7 +114,8 @@ def _rows_rel(bl, a, b):
 
 
 @pytest.mark.parametrize("kind", ["fp64", "mixed"])
-@pytest.mark.parametrize("psi4,row", [(False, 12), (False, 1), (True, 18), (True, 12), (True, 6)])
+@pytest.mark.parametrize("psi4,row", [(False, 12), (False, 1), (False, 3), (True, 18), (True, 12), (True, 3),
+                                       (True, 6)])
 def test_constraints_over_inputs(kind, psi4, row, monkeypatch):
     """Over rows that the constraints read (gt, At, chi to Gt) in several
     launches, and over rows that they do not (shift and B): the values of
