@@ -74,7 +74,7 @@ def generate_groups(write=True):
     S = bssn_rhs_stages(tails=True)
     res = {}
     for g, order in GROUPS.items():
-        E = emit_stages(S, output_order=order, barrier=False)
+        E = emit_stages(S, output_order=order, barrier=False, alt_early=True)
         text = HEADER.format(flops=E.flops, ntemps=E.ntemps, ninputs=len(E.inputs)) + TAIL_NOTE + E.text
         if write:
             with open(os.path.join(ROOT, f"sympygr_amd/csrc/gen/bssn_algebra_{g}.inc"), "w") as f:

@@ -120,7 +120,8 @@ class Emitted:
         self.ntemps = ntemps
 
 
-def emit_stages(S, tmp_prefix="t_", indent="    ", output_order=None, barrier=False) -> Emitted:
+def emit_stages(S, tmp_prefix="t_", indent="    ", output_order=None, barrier=False,
+                alt_early=False) -> Emitted:
     names = []
     exprs = []
     for _, pairs in S.stages:
@@ -184,20 +185,12 @@ def emit_stages(S, tmp_prefix="t_", indent="    ", output_order=None, barrier=Fa
         for s in names:
             emit(s)
     order = output_order or list(range(len(out_names)))
-    for oi in order:
-        n, e = out_names[oi], out_reduced[oi]
-        for fs in sorted(e.free_symbols, key=lambda x: x.name):
-            if fs in defs:
-                emit(fs)
-        load_inputs(e)
-        flops += count_flops(e)
-        lines.append(f"{indent}BSSN_OUT({oi}, {printer.doprint(e)});")
-        if barrier:
-            lines.append(f"{indent}BSSN_BARRIER();")
-    # alternative-gauge values of this group's outputs, in one block at the
-    # end: their extra inputs are loaded only when that gauge is on
     alts = [oi for oi in order if oi in alt_reduced]
-    if alts:
+
+    def emit_alternatives():
+        """Alternative-gauge values of this group's outputs, in one block:
+        their extra inputs are loaded only when that gauge is on."""
+        nonlocal flops, indent
         outer = indent
         indent = outer + "    "
         saved_loaded, saved_emitted = set(loaded), set(emitted)
@@ -210,9 +203,39 @@ def emit_stages(S, tmp_prefix="t_", indent="    ", output_order=None, barrier=Fa
             load_inputs(ea)
             flops += count_flops(ea)
             lines.append(f"{indent}BSSN_OUT_ALT({oi}, {printer.doprint(ea)});")
+        indent = outer
         lines.append(f"{outer}}}")
         loaded.clear()
         loaded.update(saved_loaded)
         emitted.clear()
         emitted.update(saved_emitted)
+
+    # alt_early: the alternatives stand before the first output of a field that
+    # they read (its array may be the input array); the including unit then
+    # does not store the outputs that they replace.  Else at the end, where
+    # they replace what was stored.
+    alt_reads = set()
+    todo = [fs for e in alt_reduced.values() for fs in e.free_symbols]
+    while todo:
+        fs = todo.pop()
+        if fs in defs:
+            todo.extend(defs[fs].free_symbols)
+        elif (classify_input(fs.name) or ("", "", 0))[0] == "U":
+            alt_reads.add(FIELD_INDEX[classify_input(fs.name)[1]])
+    pending = bool(alts)
+    for oi in order:
+        if pending and alt_early and oi in alt_reads:
+            emit_alternatives()
+            pending = False
+        n, e = out_names[oi], out_reduced[oi]
+        for fs in sorted(e.free_symbols, key=lambda x: x.name):
+            if fs in defs:
+                emit(fs)
+        load_inputs(e)
+        flops += count_flops(e)
+        lines.append(f"{indent}BSSN_OUT({oi}, {printer.doprint(e)});")
+        if barrier:
+            lines.append(f"{indent}BSSN_BARRIER();")
+    if pending:
+        emit_alternatives()
     return Emitted("\n".join(lines) + "\n", flops, inputs, len(emitted))

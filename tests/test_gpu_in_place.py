@@ -156,3 +156,20 @@ def test_constraints_over_inputs_refused_if_a_block_does_not_fit(monkeypatch):
     plan.constraints(over, over[8:12])
     torch.cuda.synchronize()
     assert _rows_rel(bl, over[8:12], sep) <= 1e-11
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_rochester_rhs_in_place(precision, monkeypatch):
+    """The Rochester shift equation reads Gt at the point: before its own
+    output is stored over it.  The bits of separate arrays (same kernels)."""
+    import torch
+    import sympygr_amd as sgr
+    bl, u, _ = _tiling("fp64")
+    prm = sgr.params(adv="upwind", ko_sigma=0.1, gauge="rochester", xi=(1, 1, 1), precision=precision)
+    for pipe in (None, "5"):
+        plan = _plan(bl, prm, monkeypatch, pipe)
+        sep, got = u.clone(), u.clone()
+        plan.rhs(sep, u)
+        plan.rhs(got, got)
+        torch.cuda.synchronize()
+        assert torch.equal(got, sep)
