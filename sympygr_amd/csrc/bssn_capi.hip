@@ -340,6 +340,14 @@ std::vector<uint8_t> closure_tiles(const std::vector<BlockDesc> &hb, const std::
     return slow;
 }
 
+// Whether a tile's last point lies within 4 GiB of its first in a field array,
+// the reach of k_rhs's stores (planes of less than 76 million nodes for 8^3).
+bool stores_reach(const BlockDesc &d)
+{
+    const uint64_t row = (uint64_t)d.n[0], plane = row * d.n[1];
+    return 8 * ((d.tdim[2] - 1) * plane + (d.tdim[1] - 1) * row + d.tdim[0]) < 0xFFFFFFF0ull;
+}
+
 // The list of one k_rhs launch over tiles t0 .. t0 + n - 1: eight consecutive
 // ranges of about equal cost (CLOSURE_COST: measured ratio of the two kinds of
 // tiles), in each the tiles without closure forms first.  Appends to `order`.
@@ -693,7 +701,8 @@ int sgr_plan_create(sgr_plan **plan, const sgr_block *blocks, uint32_t nblocks, 
         p->all[0] = tile_list(slow, 0, p->nfast, order);
         p->all[1] = tile_list(slow, p->nfast, p->ntiles - p->nfast, order);
     }
-    if (one_pass(*params) && p->ntiles) {
+    // (none: every call takes the two passes)
+    if (one_pass(*params) && p->ntiles && std::all_of(p->hblocks.begin(), p->hblocks.end(), stores_reach)) {
         const uint64_t nc = (p->ntiles + p->chunk_tiles - 1) / p->chunk_tiles;
         if (nc == 1) p->lists.push_back(p->all);
         for (uint64_t c = 0; nc > 1 && c < nc; c++) {
@@ -815,7 +824,7 @@ int sgr_plan_get_info(const sgr_plan *plan, sgr_plan_info *info)
     info->derivative_slots = rs_nslot(plan->nf) + plan->nf;
     info->chunks = plan->chunk_tiles ? (plan->ntiles + plan->chunk_tiles - 1) / plan->chunk_tiles : 0;
     info->pipelined = plan->pipe && info->chunks > 1;
-    info->tile_queue = plan->use_queue && !one_pass(plan->params);
+    info->tile_queue = plan->use_queue && plan->lists.empty();
     return SGR_OK;
 }
 

@@ -676,8 +676,8 @@ __device__ __forceinline__ void one_pass(const FieldPtrs &in, const OutPtrs &out
         // wait for the next field's loads is one for the last field's stores too: 512 x
         // 32^3 7.49 -> 7.28 ms, CCZ4 3% (general shapes 11%).  The general BSSN kernels
         // spill scalar registers over it (33^3 blocks 1.36 -> 1.55 ms) and keep the
-        // branch.  (32 bits of offset: in and out arrays of a block with larger planes
-        // fit no device.)
+        // branch.  (32 bits of offset: a plan with larger planes has no tile lists,
+        // stores_reach.)
         constexpr bool MASKED = !GEN || (CCZ4 && !RK);
         const uint64_t corner = tc.i0 + (uint64_t)n0 * (tc.j0 + (uint64_t)n1 * tc.k0);
         uint32_t soff;
