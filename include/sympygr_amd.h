@@ -109,9 +109,10 @@ typedef struct sgr_plan sgr_plan;
 
 typedef struct {
     uint64_t blocks;
-    uint64_t tiles;              /* RHS work tiles: 8^3, or the shape tuned for the block's
-                                    size (the library's tile table; SGR_TILE_SHAPE=tx,ty,tz
-                                    forces one shape on every block) */
+    uint64_t tiles;              /* RHS work tiles: 8^3, or another shape for the block's
+                                    size (by the tile count in one-pass plans, by the
+                                    library's tile table in two-pass plans;
+                                    SGR_TILE_SHAPE=tx,ty,tz forces one on every block) */
     uint64_t interior_points;
     uint64_t workspace_bytes;    /* device scratch held by the plan */
     uint32_t derivative_slots;   /* derivative values staged per point */
@@ -121,11 +122,11 @@ typedef struct {
                                     pointwise pass on a second stream the plan owns): plans
                                     needing more than one chunk, and plans of at least 8192
                                     tiles without the tile queues.  One-pass plans (FP64,
-                                    BSSN, standard gauge, Kreiss-Oliger) run their chunks
-                                    alternately on the two streams */
+                                    standard gauge: BSSN and CCZ4, any dissipation) run
+                                    their chunks alternately on the two streams */
     uint32_t tile_queue;         /* 1: the stencil pass is a persistent grid fed by per-XCD
-                                    tile queues (plans where at least a tenth of the tiles
-                                    reach a flagged face) */
+                                    tile queues (two-pass plans where at least a tenth of
+                                    the tiles reach a flagged face) */
 } sgr_plan_info;
 
 /* Replaces the per-block setup of the reference bssnRHS block loop
@@ -155,7 +156,7 @@ int sgr_rhs(sgr_plan *plan, double *const out[SGR_NUM_VARS], const double *const
 /* Same as sgr_rhs, and records events[0..1] around the stencil pass and
  * events[2..3] around the pointwise kernel on `stream` (hipEventElapsedTime
  * then gives each pass's duration).  A one-pass plan (FP64, standard gauge)
- * has one kernel: events[0..1] bracket it, events[2..3] are recorded after it
+ * has one kernel (in place, the two passes): events[0..1] bracket it, events[2..3] are recorded after it
  * (with TVB dissipation they bracket the pass that adds it).  For a plan that
  * runs in several workspace chunks (pipelined or not), events[0..1] bracket
  * the whole call (without that pass) and events[2..3] are recorded at its
@@ -232,8 +233,7 @@ int sgr_rk4_stage(sgr_plan *plan, int stage, double dt, const double *const u_n[
 int sgr_rk4_step(sgr_plan *plan, double dt, double *const u[SGR_NUM_VARS], double *const s_a[SGR_NUM_VARS],
                  double *const s_b[SGR_NUM_VARS], double *const acc[SGR_NUM_VARS], hipStream_t stream);
 
-/* The same step captured once into a HIP graph (4 ghost refreshes + 4 stages =
- * 20 kernel nodes) and replayed with sgr_graph_launch. */
+/* The same step captured once into a HIP graph (4 ghost refreshes + 4 stages) and replayed with sgr_graph_launch. */
 typedef struct sgr_graph sgr_graph;
 int sgr_rk4_graph_create(sgr_plan *plan, double dt, double *const u[SGR_NUM_VARS], double *const s_a[SGR_NUM_VARS],
                          double *const s_b[SGR_NUM_VARS], double *const acc[SGR_NUM_VARS], sgr_graph **graph);

@@ -43,14 +43,15 @@ struct LaunchArgs {
     bool upwind;
     bool mixed;
     TileList list[2];            // one-pass RHS: the launch's 8^3 tiles, and its others
-    bool fused;                  // RHS: the one-pass kernel (k_rhs, which needs no workspace), see fused_rhs
+    bool fused;                  // RHS: the one-pass kernel (k_rhs, which needs no workspace), see rhs_impl
     bool ccz4;                   // the CCZ4 system (25 fields) instead of BSSN
-    hipEvent_t ev[4];            // optional: start/stop of k_stencil, start/stop of k_pointwise
+    hipEvent_t ev[4];            // optional: start/stop of k_stencil, start/stop of k_pointwise; one pass:
+                                 // start/stop of k_rhs, start/stop of k_tvb_add (without TVB recorded after k_rhs)
     RkArgs rk;                   // rk.stage < 0: plain RHS
     int derivs_threads;          // constraint pass: k_derivs workgroup size, 256 or 512
     // RHS dissipation: 0 Kreiss-Oliger (in the stencil pass, params.ko_sigma),
-    // 1 TVB3, 2 TVB5 (k_tvb adds diss_sigma times it to the tails; the
-    // stencil pass then runs with params.ko_sigma = 0)
+    // 1 TVB3, 2 TVB5 (the stencil pass runs with params.ko_sigma = 0 and k_tvb
+    // adds diss_sigma times it to the tails; after k_rhs, k_tvb_add to the outputs)
     int diss;
     double diss_sigma;
     double *lam;                 // TVB: speeds along x, y, z, lam_span nodes each
@@ -72,7 +73,7 @@ hipError_t launch_ghost_fill(OutPtrs u, int nf, const GhostPatch *patches, const
 // the RHS as one kernel (k_rhs, one_pass.hip)
 hipError_t launch_one_pass(const LaunchArgs &a, hipStream_t s);
 
-// the CCZ4 RHS as one kernel (k_ccz4_rhs, one_pass_ccz4.hip)
+// the CCZ4 RHS as one kernel (k_rhs for Pass::CCZ4, one_pass_ccz4.hip)
 hipError_t launch_one_pass_ccz4(const LaunchArgs &a, hipStream_t s);
 
 // k_rhs, or k_stencil and the pointwise kernel

@@ -2,9 +2,9 @@
 //
 // The FP64 right-hand side in the standard gauge is one kernel, k_rhs
 // (one_pass.h).  Mixed precision, the Rochester gauge and calls whose outputs
-// overlap their inputs are two passes
-// over interior tiles (8x8x8, or another shape for the block's size), with a
-// tile-major derivative workspace between them:
+// share memory with their inputs are two passes over interior tiles (8x8x8, or
+// another shape for the block's size), with a tile-major derivative workspace
+// between them:
 //
 //   k_stencil    one 512-thread workgroup per tile.  Field by field, the 14^3
 //                halo tile is staged in LDS (the next field's tile in flight
@@ -26,7 +26,8 @@
 //
 // Both read the block table and a tile->block map, so one launch covers any
 // mix of block sizes.  k_derivs + k_constraints are the constraint pass of
-// calls whose outputs share memory with the inputs (the stencil kernel of the
+// calls whose outputs share memory with the inputs they read, and of two-pass
+// plans with 8^3 tiles on blocks of 7 points (the stencil kernel of the
 // earlier layout, which stages every first derivative; monitor.hip otherwise);
 // k_ghost_sep / k_ghost_copy refresh ghost nodes from the owning blocks.
 #include <hip/hip_ext.h>
