@@ -60,7 +60,9 @@ typedef struct {
     int32_t adv_mode;         /* SGR_ADV_CENTRED (as shipped: deriv64adv_* = deriv64_*)
                                  or SGR_ADV_UPWIND (deriv42adv_*, bssn/src/derivs.cpp:495-906) */
     int32_t precision;        /* SGR_PREC_FP64, or SGR_PREC_MIXED: FP64 state, stencils,
-                                 KO and boundary terms; FP32 pointwise algebra */
+                                 KO and boundary terms; FP32 pointwise algebra (two
+                                 passes: slower than FP64 in the standard gauge, which
+                                 runs one kernel) */
     /* Gauge variants the reference selects at compile time (bssn/src/rhs.cpp:224-243): */
     int32_t gauge;            /* SGR_GAUGE_STANDARD (bssneqs_eta_*_standard_gauge.cpp) or
                                  SGR_GAUGE_ROCHESTER (USE_ROCHESTER_GAUGE: GR/bssn.py:194-209,

@@ -100,7 +100,7 @@ const TileShapeEntry kTileTable[] = {
 // few: all the launch's 8^3 tiles run at once, then the time of one tile counts
 // (one block of 25^3 points as 64 8^3 tiles 160 us, as 18 larger ones 178 us).
 constexpr double GENERAL_TILE_COST = 1.35;
-constexpr uint64_t FEW_TILES = 256;  // a workgroup on every CU
+constexpr uint64_t FEW_TILES = 256;  // a workgroup on every CU of an MI355X
 uint64_t cube_tiles(const sgr_block &b)
 {
     uint64_t t = 1;

@@ -260,9 +260,9 @@ GhostTable build_ghost_table(const sgr_block *blocks, uint32_t nb)
             T.patches.push_back(g);
         }
         // boxes of one source block side by side: run together on one XCD, they
-        // find its rows in that XCD's L2 (848 leaves: a third less read, 6.07 ->
-        // 5.82 ms; what bounds the refresh is memory traffic by whole lines for
-        // ghost layers three nodes deep)
+        // find its rows in that XCD's L2.  Octrees of 288, 848 and 1464 leaves:
+        // 2.32 -> 2.18, 6.06 -> 5.82, 10.1 -> 9.4 ms; 848 leaves read 22.1 ->
+        // 14.9 GB (counted) and write 5.2, so reads are no longer what bounds it
         std::stable_sort(T.boxes.begin() + T.bstart[c], T.boxes.end(), [&](const GhostBox &a, const GhostBox &b) {
             return T.patches[a.patch].src_off < T.patches[b.patch].src_off;
         });
